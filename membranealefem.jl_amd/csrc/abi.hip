@@ -51,7 +51,7 @@ void free_all(Ctx &c) {
                   c.d_red,  c.d_csc_src, c.d_csc_val, c.d_eq,     c.d_band,   c.d_linv,
                   c.d_uinv, c.d_piv,  c.d_V,       c.d_Z,       c.d_h,      c.d_coef,
                   c.d_mdot_part, c.d_t2, c.d_presc_idx, c.d_presc_val, c.d_s1, c.d_s2,
-                  c.d_sweep_err, c.d_pf_el, c.d_pf_slot, c.d_pf_rel, c.d_pf_out,
+                  c.d_sweep_err, c.d_pf_el, c.d_pf_slot, c.d_pf_rel,
                   c.d_obel, c.d_crnr, c.d_out, c.d_amax, c.d_tw_z, c.d_tw_br,
                   c.d_tw_cr, c.d_tw_dr, c.d_tw_s1, c.d_tw_s2, c.d_pub, c.d_span};
   for (void *p : ptrs)
@@ -65,10 +65,10 @@ void free_all(Ctx &c) {
 
 }  // namespace
 
-// Device copies of the pull-force maps and its output buffers (first use).
+// Device copies of the pull-force maps and its residual buffer (first use).
 // Callers check c.pf_err first; HIP failures throw HipError.
 void mafem::ensure_pull(Ctx &c) {
-  if (c.d_pf_out || !c.pf_err.empty()) return;
+  if (c.pf_ready || !c.pf_err.empty()) return;
   std::lock_guard<std::mutex> no_capture(capture_mutex());
   const size_t n = c.h_pf_el.size();
   MAFEM_HIP(hipMalloc((void **)&c.d_pf_el, sizeof(int32_t) * n));
@@ -76,7 +76,7 @@ void mafem::ensure_pull(Ctx &c) {
   MAFEM_HIP(hipMalloc((void **)&c.d_pf_rel, sizeof(double) * n * c.ne));
   MAFEM_HIP(hipMemcpy(c.d_pf_el, c.h_pf_el.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
   MAFEM_HIP(hipMemcpy(c.d_pf_slot, c.h_pf_slot.data(), n * 9, hipMemcpyHostToDevice));
-  MAFEM_HIP(hipMalloc((void **)&c.d_pf_out, sizeof(double) * 6));
+  c.pf_ready = true;
 }
 
 namespace {
@@ -680,7 +680,7 @@ double linear_solve(Ctx &c, const double *d_b, double *d_x) {
 // ------------------------------------------------ allocation-free pull force
 //
 // Scratch of mafem_pull_force_noalloc: the adjacent-element list, the node
-// slot maps, the adjacent elements' residuals and the 6 outputs.  Each device
+// slot maps and the adjacent elements' residuals.  Each device
 // the library runs on holds one copy until the process ends, shared by every
 // call on that device (calls that overlap on one device race).  Host code
 // never passes `scratch` itself to a kernel or copy: its name is a host-side
@@ -689,12 +689,10 @@ double linear_solve(Ctx &c, const double *d_b, double *d_x) {
 constexpr size_t kScratchBytes = 64 * 1024;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-constexpr int kMaxAdj = 25;  // (2 poly + 1)^2 adjacent elements for poly = 2
-
 struct PullMaps {
   int32_t n;
-  int32_t el[kMaxAdj];
-  int8_t slot[9 * kMaxAdj];
+  int32_t el[MAX_ADJ];
+  int8_t slot[9 * MAX_ADJ];
 };
 
 __global__ void k_stage_pull_maps(PullMaps m, int32_t *__restrict__ el, int8_t *__restrict__ slot) {
@@ -1066,9 +1064,9 @@ int mafem_pull_force(mafem_ctx *ctx, double *x_pull, double *f_pull) {
     if (c.motion == STATIC) return fail(c, "f_pull needs 3-D velocity", MAFEM_EINVAL);
     MAFEM_HIP(hipSetDevice(c.dev));
     ensure_pull(c);
-    launch_pull_force(c, c.stream, c.d_pf_el, c.d_pf_slot, c.d_pf_rel, c.d_pf_out);
-    MAFEM_HIP(hipMemcpyAsync(c.h_red, c.d_pf_out, sizeof(double) * 6, hipMemcpyDeviceToHost,
-                             c.stream));
+    // the six outputs go straight to pinned host memory (a copy of 48 bytes costs
+    // more than the kernel that forms them)
+    launch_pull_force(c, c.stream, c.d_pf_el, c.d_pf_slot, c.d_pf_rel, c.h_red);
     MAFEM_HIP(hipStreamSynchronize(c.stream));
     for (int k = 0; k < 3; ++k) {
       x_pull[k] = c.h_red[k];
@@ -1084,9 +1082,9 @@ int mafem_pull_force_noalloc(mafem_ctx *ctx, double *x_pull, double *f_pull) {
     if (!c.pf_err.empty()) return fail(c, c.pf_err, MAFEM_EINVAL);
     if (c.motion == STATIC) return fail(c, "f_pull needs 3-D velocity", MAFEM_EINVAL);
     const int64_t n = (int64_t)c.h_pf_el.size();
-    // scratch layout: el[n] at 0, slot[9 n] at 128, rel[n ne] at 384, out[6] after it
-    const size_t need = 384 + sizeof(double) * ((size_t)n * c.ne + 6);
-    if (n > kMaxAdj || need > kScratchBytes)
+    // scratch layout: el[n] at 0, slot[9 n] at 128, rel[n ne] at 384
+    const size_t need = 384 + sizeof(double) * (size_t)n * c.ne;
+    if (n > MAX_ADJ || need > kScratchBytes)
       return fail(c,
                   "pull force scratch: " + std::to_string(need) + " bytes needed, " +
                       std::to_string(kScratchBytes) + " available (" + std::to_string(n) +
@@ -1097,15 +1095,13 @@ int mafem_pull_force_noalloc(mafem_ctx *ctx, double *x_pull, double *f_pull) {
     int32_t *el = (int32_t *)base;
     int8_t *slot = (int8_t *)(base + 128);
     double *rel = (double *)(base + 384);
-    double *out = rel + (size_t)n * c.ne;
     PullMaps m{};
     m.n = (int32_t)n;
     for (int64_t k = 0; k < n; ++k) m.el[k] = c.h_pf_el[k];
     for (int64_t k = 0; k < 9 * n; ++k) m.slot[k] = c.h_pf_slot[k];
     hipLaunchKernelGGL(k_stage_pull_maps, dim3(1), dim3(256), 0, c.stream, m, el, slot);
     MAFEM_HIP(hipGetLastError());
-    launch_pull_force(c, c.stream, el, slot, rel, out);
-    MAFEM_HIP(hipMemcpyAsync(c.h_red, out, sizeof(double) * 6, hipMemcpyDeviceToHost, c.stream));
+    launch_pull_force(c, c.stream, el, slot, rel, c.h_red);
     MAFEM_HIP(hipStreamSynchronize(c.stream));
     for (int k = 0; k < 3; ++k) {
       x_pull[k] = c.h_red[k];

@@ -85,9 +85,9 @@ struct Geo {
   N idet;           // 1 / det a_{αβ}
 };
 
-// Passes of the area kernel.  PLAIN: dual numbers throughout.  PRIMAL: one
-// lane per (element, Gauss point) evaluates the point's values in real
-// arithmetic and keeps them in LDS (slots below).  TANGENT: the lanes of the
+// Passes of the area kernel.  PLAIN: dual numbers throughout (the edges'
+// geometry).  PRIMAL: one lane per (element, Gauss point) evaluates the
+// point's values in real arithmetic and keeps them in LDS (slots below).  TANGENT: the lanes of the
 // tangent columns take those values as the value parts of their dual numbers,
 // so only the derivative parts are computed per column (sums over the nine
 // nodes, quotients and the square root of the metric are not repeated).
@@ -169,7 +169,7 @@ __device__ __forceinline__ void geometry(const double *X /*[3][9]*/, const doubl
 
 // One Gauss point of the area element (GeoDynStress.jl:111-159,
 // FiniteElement.jl:284-313).  PRIMAL ends after the stresses, with the point's
-// values in pr; PLAIN and TANGENT add the lane's rows (nodes a_lo .. a_lo +
+// values in pr; TANGENT adds the lane's rows (nodes a_lo .. a_lo +
 // NPP - 1) of the tangent column to acc and its own row's residual to racc.
 template <int MO, class N, int PS, int P, int NR>
 __device__ __forceinline__ void gp_eval(const double *X, const double *C, const double *rec,
@@ -410,31 +410,26 @@ __device__ __forceinline__ void gp_eval(const double *X, const double *C, const 
   }
 }
 
-// LIST = false: elements 0..numel-1, outputs K_el and r_el per element, in
-// two passes (PRIMAL, then TANGENT).  LIST = true: the numel elements
-// elist[0..numel-1], output r_el only, at the element's position in the list
-// (PLAIN: the tangents are dead code there).  P lanes share each tangent
-// column (lane part p takes the rows of nodes p NPP .. p NPP + NPP - 1, NPP =
-// ceil(9 / P)); the part holding the column's own row writes its r_el entry.
-template <int MO, bool LIST = false, int P = LIST ? 1 : Lay<MO>::PARTS>
+// K_el and r_el of the block's elements in two passes (PRIMAL, then TANGENT).
+// P lanes share each tangent column (lane part p takes the rows of nodes p NPP
+// .. p NPP + NPP - 1, NPP = ceil(9 / P)); the part holding the column's own
+// row writes its r_el entry.
+template <int MO, int P = Lay<MO>::PARTS>
 __device__ __forceinline__ void area_body(
     int64_t bid, int64_t numel, int64_t numnp, const int32_t *__restrict__ ix,
     const int32_t *__restrict__ uel, const uint8_t *__restrict__ active,
     const double *__restrict__ xms, const double *__restrict__ cps,
     const double *__restrict__ ufns, const double *__restrict__ dbt, PhysParams ph,
-    double dt, double *__restrict__ kel, double *__restrict__ rel,
-    const int32_t *__restrict__ elist = nullptr) {
+    double dt, double *__restrict__ kel, double *__restrict__ rel) {
   using L = Lay<MO>;
-  auto EL = [&](int64_t i) -> int64_t { return LIST ? (int64_t)elist[i] : i; };
   constexpr int NDF = L::NDF, NE = L::NE;
   constexpr int NPP = (9 + P - 1) / P, NR = NPP * NDF, LPE = NE * P;
   constexpr int MAXE = 256 / LPE + 2;  // elements a 256-lane block can touch
-  constexpr bool STAGED = !LIST;
   constexpr int NS = L::HAS_VM ? N_SLOTS : S_VM;  // slots this motion uses
   __shared__ double sX[MAXE][3 * 9];
   __shared__ double sC[MAXE][NDF * 9];
   __shared__ double sB[MAXE][9 * RECP];
-  __shared__ double sP[STAGED ? MAXE * 9 : 1][STAGED ? NS : 1];
+  __shared__ double sP[MAXE * 9][NS];
 
   const int64_t f0 = bid * 256;
   const int64_t e_lo = f0 / LPE;
@@ -445,7 +440,7 @@ __device__ __forceinline__ void area_body(
   for (int k = threadIdx.x; k < nle * 9 * (3 + NDF); k += 256) {
     const int le = k / (9 * (3 + NDF)), rem = k % (9 * (3 + NDF));
     const int comp = rem / 9, a = rem % 9;
-    const int64_t node = ix[EL(e_lo + le) * 9 + a];
+    const int64_t node = ix[(e_lo + le) * 9 + a];
     if (comp < 3)
       sX[le][comp * 9 + a] = xms[node + numnp * comp];
     else
@@ -454,34 +449,31 @@ __device__ __forceinline__ void area_body(
   // stage the 9 Gauss-point basis records of each element
   for (int k = threadIdx.x; k < nle * 9 * RECP; k += 256) {
     const int le = k / (9 * RECP), rem = k % (9 * RECP);
-    sB[le][rem] = ufns[(int64_t)uel[EL(e_lo + le)] * 9 * RECP + rem];
+    sB[le][rem] = ufns[(int64_t)uel[e_lo + le] * 9 * RECP + rem];
   }
   __syncthreads();
 
   const double azv = ph.adb / ph.zv;
-  if constexpr (STAGED) {
-    // primal pass: one lane per (element, Gauss point) of the block
-    for (int k = threadIdx.x; k < nle * 9; k += 256) {
-      const int le = k / 9, gp = k % 9;
-      double none[1];
-      double rnone = 0.0;
-      gp_eval<MO, R, PRIMAL, 1, 1>(sX[le], sC[le], &sB[le][gp * RECP], 0, -1, -1, 0, -1, 0.0,
-                                   0.0, ph, azv, sP[k], none, rnone);
-    }
-    __syncthreads();
+  // primal pass: one lane per (element, Gauss point) of the block
+  for (int k = threadIdx.x; k < nle * 9; k += 256) {
+    const int le = k / 9, gp = k % 9;
+    double none[1];
+    double rnone = 0.0;
+    gp_eval<MO, R, PRIMAL, 1, 1>(sX[le], sC[le], &sB[le][gp * RECP], 0, -1, -1, 0, -1, 0.0, 0.0,
+                                 ph, azv, sP[k], none, rnone);
   }
+  __syncthreads();
 
   const int64_t f = f0 + threadIdx.x;
   const bool valid = f < numel * LPE;
   const int64_t e = valid ? f / LPE : e_hi;
-  const int64_t eg = EL(e);
   const int part = (int)(f % LPE) / NE;
   const int col = (int)(f % NE);
   const int a_lo = part * NPP;  // first node of this lane's rows
   const int le = (int)(e - e_lo);
   const int a0 = col / NDF, d0 = col % NDF;
   const bool own_row = a0 >= a_lo && a0 < a_lo + NPP;
-  const int64_t node0 = ix[eg * 9 + a0];
+  const int64_t node0 = ix[e * 9 + a0];
   const bool act = active[d0 + NDF * node0] != 0;
   const double sC0 = act ? 1.0 : 0.0;
   const bool mot = (L::MOT0 >= 0) && d0 >= L::MOT0 && d0 < L::MOT0 + 3;
@@ -494,18 +486,13 @@ __device__ __forceinline__ void area_body(
   for (int k = 0; k < NR; ++k) acc[k] = 0.0;
   double racc = 0.0;
 
-  for (int gp = 0; gp < 9; ++gp) {
-    if constexpr (STAGED)
-      gp_eval<MO, D, TANGENT, P>(sX[le], C, &sB[le][gp * RECP], a0, d0, i0, a_lo, col, sX0,
-                                   sC0, ph, azv, sP[le * 9 + gp], acc, racc);
-    else
-      gp_eval<MO, D, PLAIN, P>(sX[le], C, &sB[le][gp * RECP], a0, d0, i0, a_lo, col, sX0, sC0,
-                                 ph, azv, nullptr, acc, racc);
-  }
+  for (int gp = 0; gp < 9; ++gp)
+    gp_eval<MO, D, TANGENT, P>(sX[le], C, &sB[le][gp * RECP], a0, d0, i0, a_lo, col, sX0, sC0, ph,
+                               azv, sP[le * 9 + gp], acc, racc);
 
   // Dohrmann--Bochev projection (FiniteElement.jl:315-327): linear in λ, p^m
   {
-    const double *T = dbt + (int64_t)uel[eg] * 81;
+    const double *T = dbt + (int64_t)uel[e] * 81;
     if (d0 == L::LAMI && act) {
 #pragma unroll
       for (int j = 0; j < NPP; ++j)
@@ -526,15 +513,13 @@ __device__ __forceinline__ void area_body(
   }
 
   if (valid) {
-    if constexpr (!LIST) {
-      double *K = kel + e * (int64_t)NE * NE;
+    double *K = kel + e * (int64_t)NE * NE;
 #pragma unroll
-      for (int j = 0; j < NPP; ++j)
-        if (9 % P == 0 || a_lo + j < 9) {
+    for (int j = 0; j < NPP; ++j)
+      if (9 % P == 0 || a_lo + j < 9) {
 #pragma unroll
-          for (int r = 0; r < NDF; ++r) K[((a_lo + j) * NDF + r) * NE + col] = acc[j * NDF + r];
-        }
-    }
+        for (int r = 0; r < NDF; ++r) K[((a_lo + j) * NDF + r) * NE + col] = acc[j * NDF + r];
+      }
     if (own_row) rel[e * NE + col] = racc;
   }
 }
@@ -659,7 +644,7 @@ __global__ __launch_bounds__(256) void k_area(
     const double *__restrict__ xms, const double *__restrict__ cps,
     const double *__restrict__ ufns, const double *__restrict__ dbt, PhysParams ph,
     double dt, double *__restrict__ kel, double *__restrict__ rel) {
-  area_body<MO, false, P>(blockIdx.x, numel, numnp, ix, uel, active, xms, cps, ufns, dbt, ph, dt,
+  area_body<MO, P>(blockIdx.x, numel, numnp, ix, uel, active, xms, cps, ufns, dbt, ph, dt,
                           kel, rel);
 }
 
@@ -674,43 +659,101 @@ __global__ __launch_bounds__(256) void k_edge(
                 kel, rel);
 }
 
-// Residuals of a list of area elements (the pull force's adjacent elements).
-template <int MO>
-__global__ __launch_bounds__(256) void k_area_list(
-    int64_t n, int64_t numnp, const int32_t *__restrict__ ix, const int32_t *__restrict__ uel,
-    const uint8_t *__restrict__ active, const double *__restrict__ xms,
-    const double *__restrict__ cps, const double *__restrict__ ufns,
-    const double *__restrict__ dbt, PhysParams ph, const int32_t *__restrict__ elist,
-    double *__restrict__ rel) {
-  area_body<MO, true>(blockIdx.x, n, numnp, ix, uel, active, xms, cps, ufns, dbt, ph, 0.0, nullptr,
-                      rel, elist);
+// Velocity rows of the residuals of a list of area elements (the pull force's
+// adjacent elements), one block per element: nine lanes evaluate the Gauss
+// points in real arithmetic (the area kernel's PRIMAL pass), then one lane per
+// (node, Gauss point) forms its three rows and one per row sums them over the
+// points in order.  The velocity rows do not depend on the motion: every
+// formulation stages its velocities and tension (column lam) in LAG's layout.
+// 25 elements leave the chip idle, so the time is the longest lane's chain:
+// one Gauss point here, 6.9 us of kernel, against nine points of dual numbers
+// per lane when the tangent's column lanes served the list (34 us).
+__global__ __launch_bounds__(128) void k_pull_rows(
+    int64_t numnp, int ndf, int lam, const int32_t *__restrict__ ix,
+    const int32_t *__restrict__ uel, const double *__restrict__ xms,
+    const double *__restrict__ cps, const double *__restrict__ ufns, PhysParams ph,
+    const int32_t *__restrict__ elist, double *__restrict__ rel) {
+  constexpr int NS = S_VM;
+  __shared__ double sX[27], sC[36], sB[9 * RECP], sP[9][NS], sR[9][27];
+  const int t = (int)threadIdx.x;
+  const int64_t e = elist[blockIdx.x];
+  if (t < 63) {
+    const int comp = t / 9;
+    const int64_t node = ix[e * 9 + t % 9];
+    if (comp < 3) sX[t] = xms[node + numnp * comp];
+    else sC[t - 27] = cps[node + numnp * (comp < 6 ? comp - 3 : lam)];
+  }
+  for (int k = t; k < 9 * RECP; k += 128) sB[k] = ufns[(int64_t)uel[e] * 9 * RECP + k];
+  __syncthreads();
+  if (t < 9) {
+    double none[1], rnone = 0.0;
+    gp_eval<LAG, R, PRIMAL, 1, 1>(sX, sC, &sB[t * RECP], 0, -1, -1, 0, -1, 0.0, 0.0, ph, 0.0,
+                                  sP[t], none, rnone);
+  }
+  __syncthreads();
+  if (t < 81) {
+    const int gp = t / 9, a = t % 9;
+    const double *rec = &sB[gp * RECP], *pr = sP[gp];
+    const double wJ = rec[0] * pr[S_J], na = rec[1 + a], n1 = rec[10 + a], n2 = rec[19 + a];
+    const double s1 = n1 * pr[S_SG] + 0.5 * n2 * pr[S_SG + 2];
+    const double s2 = n2 * pr[S_SG + 1] + 0.5 * n1 * pr[S_SG + 2];
+    double m = 0.0;
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+      m = fma(rec[28 + 9 * v + a] - (n1 * pr[S_GA0 + v] + n2 * pr[S_GA1 + v]), pr[S_MV + v], m);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      sR[gp][a * 3 + i] =
+          wJ * (pr[S_A1 + i] * s1 + pr[S_A2 + i] * s2 + pr[S_N + i] * (m - ph.pn * na));
+  }
+  __syncthreads();
+  if (t < 27) {
+    double s = 0.0;
+#pragma unroll
+    for (int gp = 0; gp < 9; ++gp) s += sR[gp][t];
+    rel[(int64_t)blockIdx.x * 9 * ndf + t / 3 * ndf + t % 3] = s;
+  }
 }
 
 // Pull force and pulled-element position (PullForce.jl:61-80,
-// Analysis.jl:81-85).  Threads 0-2: f[c] = sum over pulled nodes k of
-// (sum over adjacent elements, in order, of the v_c row of the adjacent
-// element's local node that is pulled node k).  Threads 3-5: mean of xms over
-// the pulled element's 9 nodes.
-__global__ void k_pull_reduce(int n, int ne, int ndf, const int8_t *__restrict__ slot,
-                              const double *__restrict__ rel, const int32_t *__restrict__ pull_ix,
-                              const double *__restrict__ xms, int64_t numnp,
-                              double *__restrict__ out) {
-  const int t = threadIdx.x;
-  if (t < 3) {
-    double f = 0.0;
-    for (int k = 0; k < 9; ++k) {
-      double s = 0.0;
-      for (int q = 0; q < n; ++q)
-        for (int a = 0; a < 9; ++a)
-          if (slot[q * 9 + a] == k) s += rel[(int64_t)q * ne + a * ndf + t];
-      f += s;
-    }
-    out[3 + t] = f;
-  } else if (t < 6) {
-    const int c = t - 3;
+// Analysis.jl:81-85): f[c] = sum over pulled nodes k of (sum over adjacent
+// elements, in order, of the v_c row of the adjacent element's local node
+// that is pulled node k), one lane per (k, c); x the mean of xms over the
+// pulled element's nine nodes.  slot is inverted in LDS first (a pulled node
+// occurs at most once per element), so a lane's chain is the element count:
+// 4.4 us, against 136 us for three lanes walking all 9 n slots per node.
+__global__ __launch_bounds__(256) void k_pull_reduce(
+    int n, int ne, int ndf, const int8_t *__restrict__ slot, const double *__restrict__ rel,
+    const int32_t *__restrict__ pull_ix, const double *__restrict__ xms, int64_t numnp,
+    double *__restrict__ out) {
+  __shared__ int8_t inv[MAX_ADJ * 9];    // local node of element q that is pulled node k, or -1
+  __shared__ double sv[MAX_ADJ * 27], sf[27], sx[27];
+  const int t = (int)threadIdx.x;
+  if (t < 9 * n) inv[t] = -1;
+  for (int k = t; k < 27 * n; k += 256) {
+    const int r = k % 27;
+    sv[k] = rel[(int64_t)(k / 27) * ne + r / 3 * ndf + r % 3];
+  }
+  if (t < 27) sx[t] = xms[pull_ix[t / 3] + numnp * (t % 3)];
+  const int sl = t < 9 * n ? slot[t] : -1;
+  __syncthreads();
+  if (sl >= 0) inv[t / 9 * 9 + sl] = (int8_t)(t % 9);
+  __syncthreads();
+  if (t < 27) {
     double s = 0.0;
-    for (int a = 0; a < 9; ++a) s += xms[pull_ix[a] + numnp * c];
-    out[c] = s / 9.0;
+    for (int q = 0; q < n; ++q) {
+      const int a = inv[q * 9 + t / 3];
+      s += a >= 0 ? sv[q * 27 + a * 3 + t % 3] : 0.0;
+    }
+    sf[t] = s;
+  }
+  __syncthreads();
+  if (t < 6) {
+    const double *v = t < 3 ? sx : sf;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) s += v[k * 3 + t % 3];
+    out[t] = t < 3 ? s / 9.0 : s;
   }
 }
 
@@ -951,20 +994,10 @@ int launch_assemble(Ctx &c, double time, double dt) {
 void launch_pull_force(Ctx &c, hipStream_t s, const int32_t *el, const int8_t *slot, double *rel,
                        double *out) {
   const int64_t n = (int64_t)c.h_pf_el.size();
-  const dim3 grid((unsigned)((n * c.ne + 255) / 256));
-#define PLIST(MO)                                                                            \
-  hipLaunchKernelGGL(k_area_list<MO>, grid, dim3(256), 0, s, n, c.numnp, c.d_ix, c.d_uel,    \
-                     c.d_active, c.d_xms, c.d_cps, c.d_ufns, c.d_dbt, c.phys, el, rel)
-  switch (c.motion) {
-    case LAG: PLIST(LAG); break;
-    case EUL: PLIST(EUL); break;
-    case ALEV: PLIST(ALEV); break;
-    case ALEVB: PLIST(ALEVB); break;
-    default: MAFEM_HIP(hipErrorInvalidValue);
-  }
-#undef PLIST
-  MAFEM_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_pull_reduce, dim3(1), dim3(64), 0, s, (int)n, c.ne, c.ndf, slot,
+  hipLaunchKernelGGL(k_pull_rows, dim3((unsigned)n), dim3(128), 0, s, c.numnp, c.ndf,
+                     (int)(c.lam_order - 1), c.d_ix, c.d_uel, c.d_xms, c.d_cps, c.d_ufns, c.phys,
+                     el, rel);
+  hipLaunchKernelGGL(k_pull_reduce, dim3(1), dim3(256), 0, s, (int)n, c.ne, c.ndf, slot,
                      (const double *)rel, c.d_ix + 9 * (int64_t)c.pf_pull_el, c.d_xms, c.numnp,
                      out);
   MAFEM_HIP(hipGetLastError());

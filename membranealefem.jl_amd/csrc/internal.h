@@ -22,6 +22,7 @@ constexpr int NEN = 9;
 constexpr int REC = 55;      // doubles per tabulated 2-D basis record
 constexpr int RECP = 56;     // padded record stride on the device
 constexpr int TILE = 64;     // band-LU tile edge
+constexpr int MAX_ADJ = 25;    // elements around the pulled one: (2 poly + 1)^2 for poly = 2
 constexpr int SOLVE_RING = 72;  // solution tiles a sweep keeps in LDS (needs tb + 1 <= this)
 // Lanes per tangent column of the area-element kernel, by Motion (STATIC 1 ..
 // ALEVB 5; index 0 unused): each lane accumulates the rows of ceil(9 / parts)
@@ -193,7 +194,7 @@ struct Ctx {
   int32_t *d_pf_el = nullptr;    // device copies, allocated on first use
   int8_t *d_pf_slot = nullptr;
   double *d_pf_rel = nullptr;    // r_el of the adjacent elements [n][ne]
-  double *d_pf_out = nullptr;    // x_pull[3], f_pull[3]
+  bool pf_ready = false;         // the device copies are complete
 
   // output sampling (Output.jl:30-118): per boundary, its elements in order as
   // (0-based element, first record in d_bufns) pairs from h_obel[2 h_boff[b]];
@@ -333,7 +334,7 @@ std::mutex &capture_mutex();
 // kernels / launchers (assemble.hip)
 int launch_assemble(Ctx &c, double time, double dt);
 // pulled-element mean position and pull force of the current state into
-// out[6], on stream s: el / slot are device copies of c.h_pf_el / c.h_pf_slot,
+// out[6] (device or pinned host memory), on stream s: el / slot are device copies of c.h_pf_el / c.h_pf_slot,
 // rel receives the adjacent elements' residuals (h_pf_el.size() x ne)
 void launch_pull_force(Ctx &c, hipStream_t s, const int32_t *el, const int8_t *slot, double *rel,
                        double *out);
