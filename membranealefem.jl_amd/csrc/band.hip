@@ -540,26 +540,6 @@ __device__ __forceinline__ int acc_row(int j) {
   return sizeof(S) == 8 ? g + 4 * j : 4 * g + j;
 }
 
-// LU with partial pivoting of the 64x64 diagonal tile by a 256-thread block.
-// The tile is in st (st[i][0..63] = row i, original order).  Rows are not
-// moved: the candidate row with the largest |a_ij| (pivot_key) is the pivot
-// of step j, and the row chosen at step j is stored as row j of the factored
-// tile (P A = L U).  Panels of 16 columns: the first wavefront holds the
-// panel's entries of every row in registers (lane = row) and runs its 16
-// pivot steps (the pivot row's entries broadcast with readlane; rows no
-// longer candidates take a zero multiplier); the panel's pivot rows then
-// solve U12 = L11^-1 A12 (one trailing column per lane), and the four
-// wavefronts subtract L21 U12 from the rows still unchosen on the matrix cores
-// (wavefront w: rows 16w..16w+15; chosen rows enter with a zero multiplier
-// and are not written).  Only the pivot steps stay on one wavefront.  The
-// factored tile goes to A in pivot order and piv[K][j] records the original
-// index of row j; prow / cand: 64 ints of LDS each (the row chosen at step j;
-// whether row i is still a candidate).
-// amax (used when PERT): static pivoting.  amax[0] holds max |K| as the bits
-// of a non-negative double; a pivot of magnitude below thr = eps max |K| (eps
-// of the storage precision: numerically zero) is replaced by +-thr (the
-// factorization is then that of a nearby matrix, and the solve finishes with
-// FGMRES) and counted in amax[1].
 // 1 / x from the hardware reciprocal and two Newton steps (within about an
 // ulp; the multipliers of the diagonal LU are scaled by it, as LAPACK's
 // unblocked LU does; 0 gives inf as division would)
@@ -592,13 +572,82 @@ __device__ __forceinline__ void pub_stage(unsigned long long *__restrict__ pub, 
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// x += m (of lane L of the 16-lane row) * y
+template <int L>
+__device__ __forceinline__ void fmac_row(double &x, double m, double y) {
+  asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+               : "+v"(x) : "v"(m), "v"(y), "n"(L));
+}
+template <int L>
+__device__ __forceinline__ void fmac_row(float &x, float m, float y) {
+  const int b = __builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x150 + L, 0xF, 0xF, true);
+  x = fmaf(__int_as_float(b), y, x);
+}
+// m's last writes end two wait states before the DPP reads that follow (the
+// compiler does not see those inside fmac_row)
+template <class S>
+__device__ __forceinline__ void settle(S (&m)[16]) {
+  asm volatile("s_nop 1" : "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3]), "+v"(m[4]), "+v"(m[5]),
+               "+v"(m[6]), "+v"(m[7]), "+v"(m[8]), "+v"(m[9]), "+v"(m[10]), "+v"(m[11]),
+               "+v"(m[12]), "+v"(m[13]), "+v"(m[14]));
+}
+template <int I, int K, class S>
+__device__ __forceinline__ void solve_step(S (&x)[16], const S (&m)[16]) {
+  if constexpr (I < 16) {
+    fmac_row<I>(x[I], m[K], x[K]);
+    solve_step<I + 1, K>(x, m);
+  }
+}
+// x <- M^-1 x for a unit lower 16 x 16 triangle, one right-hand side per lane:
+// lane i of every 16-lane row holds -M[i][0..14] in m
+template <int K, class S>
+__device__ __forceinline__ void unit_solve16(S (&x)[16], const S (&m)[16]) {
+  if constexpr (K < 15) {
+    solve_step<K + 1, K>(x, m);
+    unit_solve16<K + 1>(x, m);
+  }
+}
+
+// keeps a loaded value's load where it is (the compiler would move it under
+// the condition that selects the value, one LDS round trip after another)
+template <class X>
+__device__ __forceinline__ void hold(X &x) { asm volatile("" : "+v"(x)); }
+
+// LU with partial pivoting of the 64x64 diagonal tile by a 256-thread block.
+// The tile is in st (st[i][0..63] = row i, original order).  Rows are not
+// moved: the candidate row with the largest |a_ij| (pivot_key) is the pivot
+// of step j, and the row chosen at step j is stored as row j of the factored
+// tile (P A = L U).  Panels of 16 columns: the first wavefront holds the
+// panel's entries of every row in registers (lane = row) and runs its 16
+// pivot steps (the pivot row's entries broadcast with readlane; rows no
+// longer candidates take a zero multiplier).  U12 = L11^-1 A12 of the panel's
+// pivot rows follows, one trailing column per lane; lane i of each 16-lane
+// row holds row i of L11, which v_fmac_f64's row broadcast delivers at the
+// rate of a plain FMA (LDS broadcasts cost 12 cycles an entry).  Then A22 -=
+// L21 U12 on the matrix cores, 16 x 16 blocks: the next panel's column first,
+// by all four wavefronts; the columns beyond it by wavefronts 1-3 while the
+// first runs the next panel's pivot steps.  Rows chosen already enter with a
+// zero multiplier and keep their entries; every operand is loaded before it
+// is selected (a load under a condition waits for the one before it).
+// The factored tile goes to A in pivot order and piv[K][j] records the
+// original index of row j; l11: 256 entries of LDS (L11, column by column),
+// prow: 64 ints (the row chosen at step j), cand: 2 x 64 ints (whether row i
+// is still a candidate, by panel parity).
+// Measured on one tile: 34.0 k cycles (24.9 k in the pivot steps), 38.4 k with
+// U12 from LDS broadcasts and the whole trailing update between two panels.
+// amax (used when PERT): static pivoting.  amax[0] holds max |K| as the bits
+// of a non-negative double; a pivot of magnitude below thr = eps max |K| (eps
+// of the storage precision: numerically zero) is replaced by +-thr (the
+// factorization is then that of a nearby matrix, and the solve finishes with
+// FGMRES) and counted in amax[1].
 template <class S, bool PERT = false>
 __device__ __forceinline__ void diag_core_mm(int64_t K, S *__restrict__ A, int32_t *__restrict__ piv,
-                                             S (*st)[T + 1], int *prow, int *cand,
+                                             S (*st)[T + 1], S *l11, int *prow, int *cand,
                                              unsigned long long *amax = nullptr,
                                              unsigned long long *pub = nullptr) {
   using V = typename Mfma<S>::V;
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
+  const int lane = (int)threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int g = lane >> 4, cc = lane & 15;
   S thr = S(0);
   if (PERT) {
@@ -606,15 +655,46 @@ __device__ __forceinline__ void diag_core_mm(int64_t K, S *__restrict__ A, int32
     thr = (S)(rel * __longlong_as_double((long long)__hip_atomic_load(
                            amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
   }
-  int npert = 0;
-  int pos = -1;
+  int npert = 0, pos = -1;
+  // block (row block b, column block C0 / 16) -= L21 U12 of panel c0
+  auto upd = [&](int b, int c0, int C0, const int *cd_) {
+    const int row = 16 * b + cc;
+    int br[4], cw[4], cd = cd_[row];
+    S a[4], bv[4];
+    V acc, old;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      a[kk] = st[row][c0 + 4 * g + kk];
+      br[kk] = prow[c0 + 4 * g + kk];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      cw[q] = cd_[16 * b + acc_row<S>(q)];
+      old[q] = st[16 * b + acc_row<S>(q)][C0 + cc];
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) bv[kk] = st[br[kk]][C0 + cc];
+    hold(cd);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      hold(a[kk]);
+      hold(bv[kk]);
+      hold(cw[kk]);
+      acc[kk] = old[kk];
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) acc = Mfma<S>::run(cd ? -a[kk] : S(0), bv[kk], acc);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) st[16 * b + acc_row<S>(q)][C0 + cc] = cw[q] ? acc[q] : old[q];
+  };
 #pragma unroll 1
   for (int pb = 0; pb < 4; ++pb) {
     const int c0 = pb * 16;
+    int *cd_ = cand + T * (pb & 1);
     if (w == 0) {
       S r[16];
 #pragma unroll
-      for (int jj = 0; jj < 16; ++jj) r[jj] = st[lane][c0 + jj];
+      for (int k = 0; k < 16; ++k) r[k] = st[lane][c0 + k];
 #pragma unroll
       for (int jj = 0; jj < 16; ++jj) {
         const unsigned key = wave_max_u32(pivot_key(r[jj], pos < 0, lane));
@@ -627,65 +707,50 @@ __device__ __forceinline__ void diag_core_mm(int64_t K, S *__restrict__ A, int32
           npert += tiny ? 1 : 0;
         }
         if (lane == p) pos = c0 + jj;
-        const S l = (pos < 0) ? r[jj] * recip_nr(pj) : S(0);
-        if (pos < 0) r[jj] = l;
+        const S nl = (pos < 0) ? r[jj] * -recip_nr(pj) : S(0);
+        if (pos < 0) r[jj] = -nl;
         if (PERT && tiny && lane == p) r[jj] = pj;
 #pragma unroll
-        for (int k = jj + 1; k < 16; ++k) r[k] = fma(-l, lane_bcast(r[k], p), r[k]);
+        for (int k = jj + 1; k < 16; ++k) r[k] = fma(nl, lane_bcast(r[k], p), r[k]);
       }
 #pragma unroll
-      for (int jj = 0; jj < 16; ++jj) st[lane][c0 + jj] = r[jj];
-      if (pos >= c0) prow[pos] = lane;
-      cand[lane] = pos < 0 ? 1 : 0;
+      for (int k = 0; k < 16; ++k) st[lane][c0 + k] = r[k];
+      if (pos >= c0) {
+        prow[pos] = lane;
+#pragma unroll
+        for (int k = 0; k < 15; ++k) l11[k * 16 + (pos - c0)] = r[k];
+      }
+      cd_[lane] = pos < 0 ? 1 : 0;
+    } else if (pb > 0) {
+      // the previous panel's update of the column blocks beyond this panel
+      const int n = 4 * (3 - pb);
+      for (int q = w - 1; q < n; q += 3)
+        upd(q & 3, c0 - 16, c0 + 16 + 16 * (q >> 2), cand + T * ((pb - 1) & 1));
     }
     __syncthreads();
     if (pb == 3) {
       if (pub) pub_stage<S>(pub, st, prow, c0);
       break;
     }
-    if (w == 0 && lane < 48 - c0) {  // U12 = L11^-1 A12, lane = trailing column
-      const int c = c0 + 16 + lane;
+    if (w == 0) {  // U12 = L11^-1 A12, lane = trailing column (the lanes beyond: the pad column)
+      const int c = c0 + 16 + lane < T ? c0 + 16 + lane : T;
       S u[16];
+      int pr[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int ri = prow[c0 + i];
-        S acc = st[ri][c];
+      for (int i = 0; i < 16; ++i) pr[i] = prow[c0 + i];
 #pragma unroll
-        for (int ii = 0; ii < i; ++ii) acc = fma(-st[ri][c0 + ii], u[ii], acc);
-        u[i] = acc;
-      }
+      for (int i = 0; i < 16; ++i) u[i] = st[pr[i]][c];
+      S m[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[prow[c0 + i]][c] = u[i];
+      for (int k = 0; k < 15; ++k) m[k] = -l11[k * 16 + cc];
+      settle(m);
+      unit_solve16<0>(u, m);
+#pragma unroll
+      for (int i = 1; i < 16; ++i) st[pr[i]][c] = u[i];
     }
     __syncthreads();
     if (pub) pub_stage<S>(pub, st, prow, c0);  // this panel's pivot rows are final
-    {  // A22 -= L21 U12 on the matrix cores, wavefront w: rows 16w .. 16w + 15
-      const int row = 16 * w + cc;
-      const bool cd = cand[row] != 0;
-      S a[4];
-      int br[4];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const int k = 4 * g + kk;
-        a[kk] = cd ? -st[row][c0 + k] : S(0);
-        br[kk] = prow[c0 + k];
-      }
-      bool wr[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wr[j] = cand[16 * w + acc_row<S>(j)] != 0;
-#pragma unroll 1
-      for (int cb = 0; cb < 3 - pb; ++cb) {
-        const int C0 = c0 + 16 + 16 * cb;
-        V acc;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = st[16 * w + acc_row<S>(j)][C0 + cc];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) acc = Mfma<S>::run(a[kk], st[br[kk]][C0 + cc], acc);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (wr[j]) st[16 * w + acc_row<S>(j)][C0 + cc] = acc[j];
-      }
-    }
+    upd(w, c0, c0 + 16, cd_);
     __syncthreads();
   }
   if (w == 0) {
@@ -699,165 +764,178 @@ __device__ __forceinline__ void diag_core_mm(int64_t K, S *__restrict__ A, int32
   }
 }
 
+// LDS of the diagonal LU: the tile, L11 of a panel, prow and both cand arrays
+constexpr int LU_LDS = T * (T + 1) + 256 + 3 * T;
+template <class S>
+__device__ __forceinline__ int *lu_prow(S *lds) {
+  return reinterpret_cast<int *>(lds + T * (T + 1) + 256);
+}
+
 // diag_core_mm on the tile staged in the first T (T + 1) entries of an LDS
-// buffer of MM_LDS entries (its index arrays follow the tile)
+// buffer of LU_LDS entries
 template <class S, bool PERT>
 __device__ __forceinline__ void diag_mm_lds(int64_t K, S *__restrict__ A, int32_t *__restrict__ piv,
                                             S *lds, unsigned long long *amax,
                                             unsigned long long *pub = nullptr) {
   S(*st)[T + 1] = reinterpret_cast<S(*)[T + 1]>(lds);
-  int *prow = reinterpret_cast<int *>(lds + T * (T + 1));
-  diag_core_mm<S, PERT>(K, A, piv, st, prow, prow + T, amax, pub);
+  int *prow = lu_prow(lds);
+  diag_core_mm<S, PERT>(K, A, piv, st, lds + T * (T + 1), prow, prow + T, amax, pub);
 }
 
-// In-place inverses of the factors of a 64x64 diagonal tile factored by
-// diag_core_mm (row i of P A = L U at st[prow[i]]: L unit lower below the
-// diagonal, U upper), in 16 x 16 blocks.  The rows are first put in pivot
-// order.  The diagonal blocks by column sweeps in place, one row per lane
-// (wavefronts 0-1: L_bb^-1 of blocks 2w and 2w + 1, wavefronts 2-3: U_bb^-1),
-// then three rounds on the matrix cores: round r forms block row r + 1 of
-// X = L^-1, X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj, and block row 2 - r of
-// Y = U^-1, Y_ij = -Y_ii sum_{k=i+1}^{j} U_ik Y_kj, each from blocks that are
-// final (every sum is formed before any job overwrites its block).  Li and Ui
-// receive the inverses as full row-major tiles (zeros outside the triangles,
-// ones on L^-1's diagonal).  256 threads; st is overwritten.
+// 16 x 16 block operands of the matrix cores from a tile in LDS, four entries
+// a lane: as A, row lane % 16 and column acc_row(kk); as B, row acc_row(kk) and
+// column lane % 16 (an accumulator's own layout, so that a product can be the
+// next one's B operand)
 template <class S>
-__device__ __forceinline__ int k_of(int kk) {  // the k a lane group feeds in MFMA step kk
-  return acc_row<S>(kk);
+__device__ __forceinline__ void blk_a(S (&v)[4], const S (*st)[T + 1], int bi, int bj) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    v[kk] = st[16 * bi + (int)(threadIdx.x & 15)][16 * bj + acc_row<S>(kk)];
 }
+template <class S>
+__device__ __forceinline__ void blk_b(S (&v)[4], const S (*st)[T + 1], int bi, int bj) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    v[kk] = st[16 * bi + acc_row<S>(kk)][16 * bj + (int)(threadIdx.x & 15)];
+}
+// entry (r, q) of a diagonal block's unit lower or upper triangle
+template <class S>
+__device__ __forceinline__ S tri(S v, bool lower, int r, int q) {
+  return lower ? (r > q ? v : (r == q ? S(1) : S(0))) : (r <= q ? v : S(0));
+}
+template <class S>
+__device__ __forceinline__ void tri_a(S (&v)[4], bool lower) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    v[kk] = tri(v[kk], lower, (int)(threadIdx.x & 15), acc_row<S>(kk));
+}
+template <class S>
+__device__ __forceinline__ void tri_b(S (&v)[4], bool lower) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    v[kk] = tri(v[kk], lower, acc_row<S>(kk), (int)(threadIdx.x & 15));
+}
+// acc += sg A B
+template <class S, class B>
+__device__ __forceinline__ void blk_mm(typename Mfma<S>::V &acc, const S (&a)[4], const B &b, S sg) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) acc = Mfma<S>::run(sg * a[kk], b[kk], acc);
+}
+
+// Inverses of the factors of a 64x64 diagonal tile in LDS (row i of P A = L U
+// at st[prow[i]], or at st[i] when prow is null: L unit lower below the
+// diagonal, U upper), in 16 x 16 blocks: the eight diagonal blocks by
+// substitution with the row broadcast of v_fmac_f64, four to a wavefront (X =
+// L^-1 on wavefront 0, Y = U^-1 on 1); then, on the matrix cores, the
+// off-diagonal blocks of the 32 x 32 halves (X_10, X_32, Y_01, Y_23, one a
+// wavefront) and the remaining 32 x 32 block of each (16 columns a
+// wavefront), X_lower = -X_bb (L_ba X_aa).  A wavefront loads all operands of
+// a stage before its first product.  Li and Ui receive the inverses as full
+// row-major tiles (zeros outside the triangles, ones on L^-1's diagonal).  256
+// threads; st is overwritten.  10.9 k cycles a tile, against 29.8 k for
+// column sweeps in LDS and one block row a round.
 template <class S>
 __device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *__restrict__ Li,
                                             S *__restrict__ Ui) {
   using V = typename Mfma<S>::V;
-  const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
-  const int cc = lane & 15;
-  {  // rows into pivot order
-    S v[T * T / 256];
+  const int lane = (int)threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int cc = lane & 15, g = lane >> 4;
+  if (prow) {  // rows into pivot order
+    S v[T / 4];
 #pragma unroll
-    for (int it = 0; it < T * T / 256; ++it) {
-      const int e = it * 256 + (int)threadIdx.x;
-      v[it] = st[prow[e / T]][e % T];
-    }
+    for (int it = 0; it < T / 4; ++it) v[it] = st[prow[4 * it + w]][lane];
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < T * T / 256; ++it) {
-      const int e = it * 256 + (int)threadIdx.x;
-      st[e / T][e % T] = v[it];
-    }
+    for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = v[it];
     __syncthreads();
   }
-  if (lane < 32) {
-    // in place, row i = lane % 16 of block b per lane, columns in sequence
-    // (a step's reads come before its writes: one wavefront per block pair)
-    const int b0 = 16 * (2 * (w & 1) + (lane >> 4)), i = cc;
-    S *ri = &st[b0 + i][b0];
-    if (w < 2) {  // X = L_bb^-1, columns from the last: X[i][j] = -sum_{k=j+1}^{i} X[i][k] L[k][j]
-#pragma unroll 1
-      for (int j = 14; j >= 0; --j) {
-        // every operand is loaded (in bounds), the terms outside j < k < i
-        // enter as zeros: the loads issue together
-        S a[14], b[14];
+  if (w < 2) {
+    // a 16-lane row per diagonal block: lane = row of the triangle and column
+    // of its inverse; U_bb with rows and columns reversed (a lower triangle
+    // too) and its rows scaled to a unit diagonal
+    const int b0 = 16 * g, rr = w == 0 ? cc : 15 - cc;
+    const S *row = &st[b0 + rr][b0];
+    S m[16], x[16];
 #pragma unroll
-        for (int k = 1; k < 15; ++k) {
-          a[k - 1] = ri[k];
-          b[k - 1] = st[b0 + k][b0 + j];
-        }
-        const S lij = ri[j];
-        S acc0 = i > j ? lij : S(0), acc1 = S(0);  // k = i: X[i][i] = 1
+    for (int k = 0; k < 15; ++k) m[k] = w == 0 ? row[k] : row[15 - k];
+    const S d = row[rr], sc = w == 0 ? S(1) : S(1) / d;
 #pragma unroll
-        for (int k = 1; k < 15; ++k) {
-          const S t = (k > j && k < i) ? a[k - 1] : S(0);
-          if (k & 1) acc1 = fma(t, b[k - 1], acc1);
-          else acc0 = fma(t, b[k - 1], acc0);
-        }
-        if (i > j) ri[j] = -(acc0 + acc1);
-      }
-    } else {  // Y = U_bb^-1, columns from the first: Y[i][j] = -Y[j][j] sum_{k=i}^{j-1} Y[i][k] U[k][j]
-#pragma unroll 1
-      for (int j = 0; j < 16; ++j) {
-        S a[15], b[15];
+    for (int k = 0; k < 15; ++k) m[k] *= -sc;
 #pragma unroll
-        for (int k = 0; k < 15; ++k) {
-          a[k] = ri[k];
-          b[k] = st[b0 + k][b0 + j];
-        }
-        const S yjj = S(1) / st[b0 + j][b0 + j];
-        S acc0 = S(0), acc1 = S(0);
+    for (int i = 0; i < 16; ++i) x[i] = i == cc ? sc : S(0);
+    settle(m);
+    unit_solve16<0>(x, m);
 #pragma unroll
-        for (int k = 0; k < 15; ++k) {
-          const S t = (k >= i && k < j) ? a[k] : S(0);
-          if (k & 1) acc1 = fma(t, b[k], acc1);
-          else acc0 = fma(t, b[k], acc0);
-        }
-        if (i < j) ri[j] = -(acc0 + acc1) * yjj;
-        else if (i == j) ri[j] = yjj;
-      }
+    for (int i = 0; i < 16; ++i) {
+      if (w == 0 && i > cc) st[b0 + i][b0 + cc] = x[i];
+      if (w == 1 && i >= cc) st[b0 + 15 - i][b0 + 15 - cc] = x[i];
     }
   }
   __syncthreads();
-  // entry (r, q) of block (bi, bj) of the tile
-  auto at = [&](int bi, int bj, int r, int q) -> S { return st[16 * bi + r][16 * bj + q]; };
-#pragma unroll 1
-  for (int rd = 0; rd < 3; ++rd) {
-    const int njob = 2 * (rd + 1);
-    V tacc[2];
+  const bool lo = w < 2;  // wavefronts 0, 1 work on X = L^-1, 2, 3 on Y = U^-1
+  {
+    // the off-diagonal blocks of the 32 x 32 halves: X_10, X_32; Y_01, Y_23
+    const int b = 2 * (w & 1), bi = lo ? b + 1 : b, bj = lo ? b : b + 1;
+    S am[4], bm[4], ad[4];
+    blk_a<S>(am, st, bi, bj);
+    blk_b<S>(bm, st, bj, bj);
+    blk_a<S>(ad, st, bi, bi);
+    __builtin_amdgcn_sched_barrier(0);
+    tri_b<S>(bm, lo);
+    tri_a<S>(ad, lo);
+    V t = V{0, 0, 0, 0}, x = t;
+    blk_mm<S>(t, am, bm, S(1));
+    blk_mm<S>(x, ad, t, S(-1));
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = w + 4 * h;
-      tacc[h] = V{0, 0, 0, 0};
-      if (q >= njob) continue;
-      // the diagonal block of the sum (X_jj unit lower, Y_jj upper) is read
-      // whole and masked
-      if (q <= rd) {  // X row i = rd + 1, column j = q: sum_{k=j}^{i-1} L_ik X_kj
-        const int i = rd + 1, j = q;
-        for (int k = j; k < i; ++k)
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            const int km = k_of<S>(kk);
-            const S a = at(i, k, cc, km), bv = at(k, j, km, cc);
-            const S b = k > j || km > cc ? bv : (km == cc ? S(1) : S(0));
-            tacc[h] = Mfma<S>::run(a, b, tacc[h]);
-          }
-      } else {  // Y row i = 2 - rd, column j = i + 1 + (q - rd - 1): sum_{k=i+1}^{j} U_ik Y_kj
-        const int i = 2 - rd, j = i + 1 + (q - rd - 1);
-        for (int k = i + 1; k <= j; ++k)
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            const int km = k_of<S>(kk);
-            const S a = at(i, k, cc, km), bv = at(k, j, km, cc);
-            const S b = k < j || km <= cc ? bv : S(0);
-            tacc[h] = Mfma<S>::run(a, b, tacc[h]);
-          }
-      }
-    }
-    __syncthreads();  // every sum is formed before any block of this round is overwritten
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = w + 4 * h;
-      if (q >= njob) continue;
-      const bool isx = q <= rd;
-      const int i = isx ? rd + 1 : 2 - rd, j = isx ? q : i + 1 + (q - rd - 1);
-      V acc = V{0, 0, 0, 0};
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const int km = k_of<S>(kk);
-        // -X_ii (unit lower) or -Y_ii (upper); the sum's accumulator row
-        // k_of(kk) of this lane's column is the B operand of step kk
-        const S d = at(i, i, cc, km);
-        const S a = isx ? (cc > km ? -d : (cc == km ? S(-1) : S(0))) : (cc <= km ? -d : S(0));
-        acc = Mfma<S>::run(a, tacc[h][kk], acc);
-      }
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) st[16 * i + acc_row<S>(jj)][16 * j + cc] = acc[jj];
-    }
-    __syncthreads();
+    for (int q = 0; q < 4; ++q) st[16 * bi + acc_row<S>(q)][16 * bj + cc] = x[q];
   }
+  __syncthreads();
+  {
+    // block column j of X (block rows 2, 3) or of Y (block rows 0, 1).  With M
+    // the factor, Z its inverse, n the block row next to the column's half and
+    // f the other one: t_i = sum_k M_ik Z_kj over the column's blocks k, z_n =
+    // -Z_nn t_n and z_f = -Z_ff t_f - Z_fn t_n
+    const int j = w, n = lo ? 2 : 1, f = lo ? 3 : 0;
+    S an[4], af[4], z[4], dn[4], df[4], off[4];
+    blk_a<S>(an, st, n, j);
+    blk_a<S>(af, st, f, j);
+    blk_b<S>(z, st, j, j);
+    blk_a<S>(dn, st, n, n);
+    blk_a<S>(df, st, f, f);
+    blk_a<S>(off, st, f, n);
+    __builtin_amdgcn_sched_barrier(0);
+    tri_b<S>(z, lo);
+    tri_a<S>(dn, lo);
+    tri_a<S>(df, lo);
+    V tn = V{0, 0, 0, 0}, tf = tn, zn = tn, zf = tn;
+    blk_mm<S>(tn, an, z, S(1));
+    blk_mm<S>(tf, af, z, S(1));
+    if (j == 0 || j == 3) {  // the column's other block: X_10 or Y_23
+      const int k = j == 0 ? 1 : 2;
+      blk_a<S>(an, st, n, k);
+      blk_a<S>(af, st, f, k);
+      blk_b<S>(z, st, k, j);
+      blk_mm<S>(tn, an, z, S(1));
+      blk_mm<S>(tf, af, z, S(1));
+    }
+    blk_mm<S>(zn, dn, tn, S(-1));
+    blk_mm<S>(zf, off, tn, S(-1));
+    blk_mm<S>(zf, df, tf, S(-1));
+    __syncthreads();  // every operand has been read
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      st[16 * n + acc_row<S>(q)][16 * j + cc] = zn[q];
+      st[16 * f + acc_row<S>(q)][16 * j + cc] = zf[q];
+    }
+  }
+  __syncthreads();
 #pragma unroll 4
   for (int it = 0; it < T * T / 256; ++it) {
-    const int e = it * 256 + (int)threadIdx.x, r = e / T, c = e % T;
-    const S v = st[r][c];
-    Li[e] = r > c ? v : (r == c ? S(1) : S(0));
-    Ui[e] = r <= c ? v : S(0);
+    const int e = it * 256 + (int)threadIdx.x, rr = e / T, c = e % T;
+    const S v = st[rr][c];
+    Li[e] = rr > c ? v : (rr == c ? S(1) : S(0));
+    Ui[e] = rr <= c ? v : S(0);
   }
 }
 
@@ -1275,48 +1353,26 @@ __global__ void k_span_init(unsigned long long *__restrict__ span) {
 
 // ------------------------------------------------- post-factorization pass
 //
-// Inverts every factored diagonal tile (one wavefront per tile, lane = column
-// of the inverse) and folds the inverses into the off-diagonal tiles,
+// Inverts every factored diagonal tile (one block per tile) and folds the inverses into the off-diagonal tiles,
 // L~_IK = L_II^-1 L_IK and U~_IJ = U_II^-1 U_IJ, so that each sweep step is a
 // single batch of tile mat-vecs: y_I = L_II^-1 P_I b_I - Σ L~_IK y_K and
 // x_I = U_II^-1 y_I - Σ U~_IJ x_J.  Every tile is independent: fully parallel.
 
-// Inverses of one factored diagonal tile by one wavefront: the tile staged in
-// LDS, L^-1 = L^-1 I and U^-1 = I U^-1 by the panel's blocked substitutions
-// (trsm_wave), so the factors are read from LDS with wave-uniform addresses.
+// inverses of one factored diagonal tile (stored in pivot order)
 template <class S>
-__device__ __forceinline__ void tile_inv_body(int64_t bid, int tb, const S *__restrict__ band,
-                                                 S *__restrict__ linv, S *__restrict__ uinv) {
-  __shared__ __align__(16) S sD[T][T];
-  __shared__ S sX[T][T + 1];
-  __shared__ S rdiag[T];
-  const int64_t I = bid;
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void tile_inv_body(int64_t I, int tb, const S *__restrict__ band,
+                                              S *__restrict__ linv, S *__restrict__ uinv) {
+  __shared__ S st[T][T + 1];
+  const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
   const S *D = tile_ptr(band, tb, I, I);
 #pragma unroll
-  for (int i = 0; i < T; ++i) sD[i][lane] = D[i * T + lane];
-#pragma unroll 8
-  for (int i = 0; i < T; ++i) sX[i][lane] = i == lane ? S(1) : S(0);
+  for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = D[(4 * it + w) * T + lane];
   __syncthreads();
-  trsm_wave<S>(0, sD, sX, rdiag);
-  __syncthreads();
-  S *Li = linv + I * (int64_t)T * T;
-#pragma unroll 8
-  for (int i = 0; i < T; ++i) Li[i * T + lane] = sX[i][lane];
-  __syncthreads();
-#pragma unroll 8
-  for (int i = 0; i < T; ++i) sX[i][lane] = i == lane ? S(1) : S(0);
-  rdiag[lane] = S(1) / sD[lane][lane];
-  __syncthreads();
-  trsm_wave<S>(1, sD, sX, rdiag);
-  __syncthreads();
-  S *Ui = uinv + I * (int64_t)T * T;
-#pragma unroll 8
-  for (int i = 0; i < T; ++i) Ui[i * T + lane] = sX[i][lane];
+  tri_inv_lds<S>(st, (const int *)nullptr, linv + I * T * T, uinv + I * T * T);
 }
 
 template <class S>
-__global__ __launch_bounds__(64) void k_tile_inv(int tb, const S *__restrict__ band,
+__global__ __launch_bounds__(256) void k_tile_inv(int tb, const S *__restrict__ band,
                                                  S *__restrict__ linv, S *__restrict__ uinv) {
   tile_inv_body<S>((int64_t)blockIdx.x, tb, band, linv, uinv);
 }
@@ -1938,7 +1994,7 @@ __global__ __launch_bounds__(256) void kb_update(StepMap sm, int64_t K, const in
 }
 
 template <class S>
-__global__ __launch_bounds__(64) void kb_tile_inv(Seg sg, const PatchDev *__restrict__ pd,
+__global__ __launch_bounds__(256) void kb_tile_inv(Seg sg, const PatchDev *__restrict__ pd,
                                                   const uint8_t *__restrict__ on,
                                                   const uint8_t *__restrict__ fac) {
   const int p = sg.map[blockIdx.x];
@@ -2110,7 +2166,7 @@ static void factor_run(Ctx &c, S *band, S *li, S *ui) {
   }
   if (c.tw_a == 0) {
     factor_chain<S, PERT>(c, c.stream, band, c.d_piv, c.d_pub, c.nt, 0, c.nt, true, true, true);
-    hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)c.nt), dim3(64), 0, c.stream, c.tb, band, li, ui);
+    hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)c.nt), dim3(256), 0, c.stream, c.tb, band, li, ui);
     hipLaunchKernelGGL(k_fold<S>, dim3((unsigned)(c.nt * (2 * c.tb + 1))), dim3(256), 0, c.stream,
                        c.nt, c.tb, band, li, ui);
     MAFEM_HIP(hipGetLastError());
@@ -2153,8 +2209,8 @@ static void factor_run(Ctx &c, S *band, S *li, S *ui) {
   factor_chain<S, PERT>(c, c.stream, band, c.d_piv, pt, rt, a, rt, true, true, false);
   // inverses of the diagonal tiles; folds: every tile row of BT, B's rows of
   // BR (its separator rows keep their raw L tiles for the solve)
-  hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)rt), dim3(64), 0, c.stream, c.tb, band, li, ui);
-  hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)nb), dim3(64), 0, c.stream, c.tb, (const S *)br,
+  hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)rt), dim3(256), 0, c.stream, c.tb, band, li, ui);
+  hipLaunchKernelGGL(k_tile_inv<S>, dim3((unsigned)nb), dim3(256), 0, c.stream, c.tb, (const S *)br,
                      li + rt * tsz, ui + rt * tsz);
   hipLaunchKernelGGL(k_fold<S>, dim3((unsigned)(rt * (2 * c.tb + 1))), dim3(256), 0, c.stream, rt,
                      c.tb, band, li, ui);
@@ -2431,7 +2487,7 @@ static void b_factor_t(BatchPlan &B, const std::vector<std::vector<StepMap>> &st
         hipLaunchKernelGGL(kb_update<S>, dim3(bu), dim3(256), 0, B.stream, smu, K, B.d_order,
                            B.d_pd, f.on, f.fac);
     }
-  hipLaunchKernelGGL(kb_tile_inv<S>, dim3(B.tiles.nblk), dim3(64), 0, B.stream, B.tiles, B.d_pd,
+  hipLaunchKernelGGL(kb_tile_inv<S>, dim3(B.tiles.nblk), dim3(256), 0, B.stream, B.tiles, B.d_pd,
                      f.on, f.fac);
   hipLaunchKernelGGL(kb_fold<S>, dim3(B.fold.nblk), dim3(256), 0, B.stream, B.fold, B.d_pd, f.on,
                      f.fac);

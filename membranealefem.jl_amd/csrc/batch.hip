@@ -258,7 +258,7 @@ void build_plan(mafem_batch &b) {
   B.vec = make_seg(b, bv, 256);
   B.node = make_seg(b, bn, 256);
   B.zero = make_seg(b, bz, 256);
-  B.tiles = make_seg(b, bt, 256);  // tile inversion (64), diagonal products (256)
+  B.tiles = make_seg(b, bt, 256);  // tile inversion, diagonal products
   B.fold = make_seg(b, bf, 256);
   std::vector<int64_t> bw(P);
   for (int p = 0; p < P; ++p) bw[p] = b.h_pd[p].sweep_w > 1 ? b.h_pd[p].sweep_w : 0;
