@@ -59,8 +59,8 @@ def pull_speed(k, total=200, final=2.0):
 # hold the runs.
 STEP_COUNTERS_KIB = {
     "k_step_la": (16013.467625473484, 19804.575757575756),
-    "knd_step_la": (3675.1130514705883, 3150.5367647058824),
-    "knd_schur": (157148.615234375, 93548.0),
+    "knd_update": None,
+    "knd_schur": None,
 }
 # the same counters per dispatch of the area kernel of the bench patch, by motion
 AREA_COUNTERS_KIB = {
@@ -792,9 +792,9 @@ def main():
 
 def nd_schur_roofline(st_list, agg):
     """The nested-dissection factorization's matrix-core kernel, knd_schur
-    (one launch per tree level: every front's boundary block minus the
-    products of its fully-summed tile rows and columns, accumulated on the
-    matrix cores and written once), which performs about three quarters of
+    (one launch per tree level: the products of every front's fully-summed
+    tile rows and columns accumulated on the matrix cores, subtracted from its
+    children's entries and written once), which performs about three quarters of
     the factorization's FLOPs.  The library times every launch on the device's
     constant clock and counts its algorithmic FLOPs ((FT - fT)^2 fT tile
     products of 2*64^3 per front) and bytes; achieved = mean FLOPs per launch /
@@ -814,8 +814,8 @@ def nd_schur_roofline(st_list, agg):
             "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
             "traffic_unit": "bytes per launch", "algorithmic_bytes": by,
             "kernel": ("knd_schur (the Schur blocks of every front of a nested-dissection "
-                       "level: boundary tiles minus the fully-summed rows' and columns' "
-                       "products, FP64 on the matrix cores)"),
+                       "level: the children's entries minus the fully-summed rows' and "
+                       "columns' products, FP64 on the matrix cores)"),
             "flops_per_launch": fl, "avg_us": us,
             "factorization_tflops": st["front_flops"] / (per_fact_us * 1e-6) / 1e12,
             "flops_per_factorization": st["front_flops"], "fronts": st["fronts"],
@@ -823,23 +823,23 @@ def nd_schur_roofline(st_list, agg):
 
 
 def nd_roofline(st_list, agg):
-    """Dominant kernel of the nested-dissection factorization, knd_step_la (one
-    launch per tile step of each tree level: for every front of the level the
-    trailing update on the matrix cores, the next 64x64 diagonal LU and the
-    next panel): the library times every launch on the device's constant clock
-    and counts its algorithmic FLOPs (per front (FT-K-1)^2 tile products of
-    2*64^3, the next diagonal LU 2/3*64^3 and 2 (FT-K-2) panel solves of
-    64^3); achieved = mean FLOPs per launch / mean launch duration, averaged
-    over the timed steps.  The whole factorization's rate is beside it."""
+    """Step kernel of the nested-dissection factorization, knd_update (one
+    launch per tile step but the last of each tree level: for every front of
+    the level the next 64x64 diagonal tile updated, factored and its factors
+    inverted, beside the products its next panel's tiles collect): the library
+    times every launch on the device's constant clock and counts its
+    algorithmic FLOPs; achieved = mean FLOPs per launch / mean launch
+    duration, averaged over the timed steps.  The whole factorization's rate
+    is beside it."""
     w = [s for s in st_list if s["step_kernel_us"] > 0]
     us = float(np.mean([s["step_kernel_us"] for s in w])) if w else float("nan")
     fl = float(np.mean([s["step_flops"] for s in w])) if w else float("nan")
     by = float(np.mean([s["step_bytes"] for s in w])) if w else float("nan")
     achieved = fl / (us * 1e-6) / 1e12
     # HBM bytes per launch from FETCH_SIZE / WRITE_SIZE per dispatch (mean
-    # over one time step's knd_step_la dispatches), scaled as for k_step_la
+    # over one time step's knd_update dispatches), scaled as for k_step_la
     traffic = None
-    counters = STEP_COUNTERS_KIB["knd_step_la"]
+    counters = STEP_COUNTERS_KIB["knd_update"]
     if counters is not None:
         traffic = (counters[0] * (131072.0 / 65545.0) + counters[1] * 1.0) * 1024.0
     st = st_list[-1]
@@ -847,9 +847,9 @@ def nd_roofline(st_list, agg):
     return {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
             "traffic_unit": "bytes per launch", "algorithmic_bytes": by,
-            "kernel": ("knd_step_la (one tile step of every front of a nested-dissection "
-                       "level: trailing update on the matrix cores, the next 64x64 diagonal "
-                       "LU and the next panel in the same launch)"),
+            "kernel": ("knd_update (one tile step of every front of a nested-dissection "
+                       "level: the next 64x64 diagonal LU with its inverses, beside the next "
+                       "panel's products on the matrix cores)"),
             "flops_per_launch": fl, "avg_us": us,
             "factorization_tflops": st["front_flops"] / (per_fact_us * 1e-6) / 1e12,
             "flops_per_factorization": st["front_flops"], "fronts": st["fronts"],

@@ -115,8 +115,8 @@ typedef struct {
                                       (trailing update, next diagonal-tile LU and next
                                       panel; band: the middle step of each factorization,
                                       nested dissection: every step launch of every
-                                      level), first block start to last block end on the
-                                      device's constant clock */
+                                      level but the last), first block start to last
+                                      block end on the device's constant clock */
   double last_relres;              /* |K du + r| / |r| of the last solve */
   int32_t sweep_groups;            /* workgroups of each triangular sweep (autotuned) */
   int32_t pivot_perturbations;     /* diagonal-tile pivots below eps max|K| (numerically
@@ -138,10 +138,10 @@ typedef struct {
   double step_bytes;               /* MAFEM_ORDER_ND: their algorithmic bytes per launch
                                       (tiles read and written once; else 0) */
   double schur_kernel_us;          /* MAFEM_ORDER_ND: mean duration of one tree level's
-                                      Schur-block launch (every front's boundary block
-                                      minus its fully-summed products), first block
-                                      start to last block end on the device's constant
-                                      clock (else 0) */
+                                      Schur-block launch (the children's boundary entries
+                                      minus every front's fully-summed products), first
+                                      block start to last block end on the device's
+                                      constant clock (else 0) */
   double schur_flops;              /* algorithmic FLOPs per such launch (per front
                                       (FT - fT)^2 fT tile products of 2*64^3) */
   double schur_bytes;              /* algorithmic bytes per such launch (each operand

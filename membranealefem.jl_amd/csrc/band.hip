@@ -501,8 +501,7 @@ __device__ __forceinline__ void tile_mm_ga(const S *__restrict__ a, const S *__r
 
 // to_lds: the updated tile goes to lds as rows of T + 1 entries (for the
 // diagonal LU that follows in the same block) instead of to the band.
-// GA: tile_mm_ga (lds of MM1_LDS entries suffices).
-template <class S, bool GA = false>
+template <class S>
 __device__ __forceinline__ void update_body(int64_t bid, int64_t K, int64_t nt, int tb, S *__restrict__ band,
                                             S *lds, bool to_lds = false) {
   const int64_t I = K + 1 + bid / tb, J = K + 1 + bid % tb;
@@ -516,8 +515,7 @@ __device__ __forceinline__ void update_body(int64_t bid, int64_t K, int64_t nt, 
 #pragma unroll
     for (int j = 0; j < 4; ++j) old[bj][j] = A[mm_row<S>(j) * T + mm_col<S>(bj)];
   S c[4][4];
-  if (GA) tile_mm_ga<S>(Lt, Ut, c, lds);
-  else tile_mm<S>(Lt, Ut, c, lds);
+  tile_mm<S>(Lt, Ut, c, lds);
   if (to_lds) {
     __syncthreads();  // every wavefront is done with the staged operands
 #pragma unroll
@@ -974,9 +972,6 @@ struct FacChain {
   int32_t fuse;
   unsigned long long *pub;  // look-ahead staging, 2 PUBW words
   int64_t k0;               // the chain's first step (its row's L tiles permuted beforehand)
-  // trailing tiles (I, J) with I, J >= s0 are not updated (a front's Schur
-  // block, which receives all its steps' products at once afterwards)
-  int64_t s0 = INT64_MAX;
 };
 
 template <class S>
@@ -1157,8 +1152,7 @@ __device__ __forceinline__ bool stage_wait(const unsigned long long *__restrict_
 // in the slot of its source row spiv[i] (each source row is read once,
 // before its slot is reused); wavefront w owns columns 16w..16w+15.  kind 1
 // (L tile, X <- X U^-1): wavefront w owns rows 16w..16w+15.  256 threads;
-// bad: an LDS int.  pub = null: sD and spiv already hold the whole factored
-// tile and its pivots (no waits; bad is not read).
+// bad: an LDS int.
 template <class S>
 __device__ __forceinline__ void staged_solve(int kind, const unsigned long long *__restrict__ pub,
                                              S (*sD)[T], S (*sX)[T + 1], S *rdiag, int *spiv,
@@ -1168,12 +1162,12 @@ __device__ __forceinline__ void staged_solve(int kind, const unsigned long long 
   const int g = lane >> 4, cc = lane & 15;
   for (int st = 0; st < 4; ++st) {
     const int s0 = 16 * st;
-    if (pub && w == 0) {
+    if (w == 0) {
       const bool ok = stage_wait<S>(pub, st, sD, spiv, err);
       if (lane == 0) *bad = ok ? 0 : 1;
     }
     __syncthreads();  // also orders the previous stage's diagonal solve before this stage
-    if (pub && *bad) return;
+    if (*bad) return;
     if (st > 0) {
       V acc;
       if (kind == 0) {  // rows s0.. (pivot order) -= L[s0.., 0..s0) Y[0..s0), columns 16w..
@@ -1239,7 +1233,6 @@ __device__ __forceinline__ void step_la_chain(int tb, const FacChain &ch, int64_
   const int64_t K = ch.K, nt = ch.nt;
   if (!ch.fuse) {
     if (bid < (int64_t)tb * tb) {
-      if (K + 1 + bid / tb >= ch.s0 && K + 1 + bid % tb >= ch.s0) return;
       update_body<S>(bid, K, nt, tb, band, lds);
     } else if (bid == (int64_t)tb * tb && K > ch.k0) {  // the deferred P_K of tile (K, K-1)
       if (threadIdx.x < T) spiv[threadIdx.x] = ch.piv[K * T + threadIdx.x];
@@ -1309,7 +1302,6 @@ __device__ __forceinline__ void step_la_chain(int tb, const FacChain &ch, int64_
   const int64_t u = r - 3 * (int64_t)tb, tm = tb - 1;
   if (u >= tm * tm) return;
   const int64_t I = K + 2 + u / tm, J = K + 2 + u % tm;
-  if (I >= ch.s0 && J >= ch.s0) return;
   update_body<S>((I - K - 1) * tb + (J - K - 1), K, nt, tb, band, lds);
 }
 
