@@ -182,3 +182,34 @@ def test_nd_panel_forms_on_every_level(monkeypatch, la, inv):
     assert rel <= 1e-9
     ref = spla.spsolve(K.tocsc(), -r)
     assert np.linalg.norm(du - ref) / np.linalg.norm(ref) <= 1e-7
+
+
+@pytest.mark.parametrize("n1,n2,precision", [(2, 9, 64), (30, 32, 64), (30, 32, 32), (34, 36, 64),
+                                             (35, 38, 64), (62, 64, 64), (66, 70, 64), (66, 70, 32)])
+def test_nd_root_widths(n1, n2, precision):
+    """ALEVB patches whose largest separator takes 1, 8, 9, 10, 16 and 17 or
+    more tile rows: one group of tile steps, a group's end at the last step,
+    and a second and third group of products in the factors and in the
+    inverses that the solve uses.  FP64 factors alone solve to the accuracy of
+    the tile-local pivoting; as an FP32 preconditioner they leave GMRES few
+    iterations."""
+    print(f"nd root width {n1}x{n2} fp{precision}", flush=True)
+    p, mesh, xms, cps = _setup(mafem.ALEVB, n1, n2)
+    dev = mafem.analysis.DeviceMesh(mesh, p)
+    try:
+        dev.set_state(xms, cps)
+        r, K = dev.assemble(1e-3, 1e-3)
+        dev.set_ordering("nd")
+        if precision == 64:
+            dev.set_solver("direct", refine_sweeps=0, rtol=1e-13)
+        else:
+            dev.set_solver("krylov", precision=32, rtol=1e-12)
+        du, rel = dev.solve(-r)
+        st = dev.stats()
+    finally:
+        dev.close()
+    true = np.linalg.norm(K @ du + r) / np.linalg.norm(r)
+    print(f"  relres {rel:.2e} ({true:.2e}), {st['front_steps']} steps, "
+          f"{st['gmres_iters']} iterations", flush=True)
+    assert true <= (1e-9 if precision == 64 else 1e-11)
+    assert precision == 64 or st["gmres_iters"] <= 60
