@@ -821,8 +821,7 @@ __device__ __forceinline__ void blk_mm(typename Mfma<S>::V &acc, const S (&a)[4]
 }
 
 // Inverses of the factors of a 64x64 diagonal tile in LDS (row i of P A = L U
-// at st[prow[i]], or at st[i] when prow is null: L unit lower below the
-// diagonal, U upper), in 16 x 16 blocks: the eight diagonal blocks by
+// at st[prow[i]]: L unit lower below the diagonal, U upper), in 16 x 16 blocks: the eight diagonal blocks by
 // substitution with the row broadcast of v_fmac_f64, four to a wavefront (X =
 // L^-1 on wavefront 0, Y = U^-1 on 1); then, on the matrix cores, the
 // off-diagonal blocks of the 32 x 32 halves (X_10, X_32, Y_01, Y_23, one a
@@ -831,7 +830,9 @@ __device__ __forceinline__ void blk_mm(typename Mfma<S>::V &acc, const S (&a)[4]
 // a stage before its first product.  Li and Ui receive the inverses as full
 // row-major tiles (zeros outside the triangles, ones on L^-1's diagonal).  256
 // threads; st is overwritten.  10.9 k cycles a tile, against 29.8 k for
-// column sweeps in LDS and one block row a round.
+// column sweeps in LDS and one block row a round and 21 k for tri_inv_sub,
+// whose smaller residuals are not worth it here, in the factorization's chain
+// (64x64 ALEVB 16.3 -> 17.6 ms a step for the same refinement sweeps).
 template <class S>
 __device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *__restrict__ Li,
                                             S *__restrict__ Ui) {
@@ -839,7 +840,7 @@ __device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *
   const int lane = (int)threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int cc = lane & 15, g = lane >> 4;
-  if (prow) {  // rows into pivot order
+  {  // rows into pivot order
     S v[T / 4];
 #pragma unroll
     for (int it = 0; it < T / 4; ++it) v[it] = st[prow[4 * it + w]][lane];
@@ -934,6 +935,129 @@ __device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *
     const S v = st[rr][c];
     Li[e] = rr > c ? v : (rr == c ? S(1) : S(0));
     Ui[e] = rr <= c ? v : S(0);
+  }
+}
+
+// v of lane row 0, 1, 2, 3 of the wavefront (16 lanes each), delivered to every
+// lane row (gfx950's row swaps: three for the four values of a 32-bit word)
+__device__ __forceinline__ void rows_all(unsigned v, unsigned (&o)[4]) {
+  const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+  o[0] = a[0];
+  o[1] = a[1];
+  o[2] = b[0];
+  o[3] = b[1];
+}
+__device__ __forceinline__ void rows_all(float v, float (&o)[4]) {
+  unsigned u[4];
+  rows_all(__float_as_uint(v), u);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) o[g] = __uint_as_float(u[g]);
+}
+__device__ __forceinline__ void rows_all(double v, double (&o)[4]) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  unsigned lo[4], hi[4];
+  rows_all((unsigned)u, lo);
+  rows_all((unsigned)(u >> 32), hi);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    o[g] = __longlong_as_double((long long)(((unsigned long long)hi[g] << 32) | lo[g]));
+}
+// accumulator row acc_row(q) of lane row g as an index into a column's 16 rows
+template <class S>
+__host__ __device__ constexpr int acc_idx(int g, int q) {
+  return sizeof(S) == 8 ? g + 4 * q : 4 * g + q;
+}
+
+// Block column J of Z = G^-1 by one wavefront, G lower triangular in 16 x 16
+// blocks with entry (i, k) at G[i si + k sk] (L itself, or U transposed) and rd
+// its diagonal's reciprocals (LOW: a unit diagonal): Z_IJ = G_II^-1 (-sum_{J <=
+// k < I} G_Ik Z_kJ).  The sums run on the matrix cores, each row's term as soon
+// as its Z_kJ is there; a diagonal block is solved by substitution
+// (unit_solve16, its rows scaled to a unit diagonal), one of Z's columns a
+// lane, every lane row alike.  Entry (i, j) of Z goes to Z[i zi + j zj], zeros
+// above the diagonal block too.
+template <class S, bool LOW>
+__device__ __forceinline__ void tri_inv_col(int J, const S *G, int si, int sk, const S *rd,
+                                            S *__restrict__ Z, int zi, int zj) {
+  using V = typename Mfma<S>::V;
+  const int cc = (int)threadIdx.x & 15, g = ((int)threadIdx.x & 63) >> 4;
+  V t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i] = V{0, 0, 0, 0};
+#pragma unroll
+  for (int I = 0; I < 4; ++I) {
+    S *out = Z + 16 * I * zi + (16 * J + cc) * zj;
+    if (I < J) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[acc_row<S>(q) * zi] = S(0);
+      continue;
+    }
+    // lane row entries: -(row cc of the unit triangle), operands of the rows below
+    const S rc = LOW ? S(1) : rd[16 * I + cc];
+    S m[16], x[16], a[3][4];
+#pragma unroll
+    for (int k = 0; k < 15; ++k) m[k] = G[(16 * I + cc) * si + (16 * I + k) * sk];
+#pragma unroll
+    for (int i = I + 1; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        a[i - 1][q] = -G[(16 * i + cc) * si + (16 * I + acc_row<S>(q)) * sk];
+#pragma unroll
+    for (int k = 0; k < 15; ++k) m[k] *= -rc;
+    if (I == J) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = i == cc ? rc : S(0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        S r4[4];
+        rows_all(LOW ? t[I][q] : t[I][q] * rd[16 * I + acc_row<S>(q)], r4);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) x[acc_idx<S>(h, q)] = r4[h];
+      }
+    }
+    settle(m);
+    unit_solve16<0>(x, m);
+    S z[4];  // rows acc_row(q): the lane's part of the result, and of a B operand
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const S lo = g & 1 ? x[acc_idx<S>(1, q)] : x[acc_idx<S>(0, q)];
+      const S hi = g & 1 ? x[acc_idx<S>(3, q)] : x[acc_idx<S>(2, q)];
+      z[q] = g & 2 ? hi : lo;
+    }
+#pragma unroll
+    for (int i = I + 1; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) t[i] = Mfma<S>::run(a[i - 1][q], z[q], t[i]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[acc_row<S>(q) * zi] = z[q];
+  }
+}
+
+// Inverses of the factors of a 64x64 diagonal tile in LDS (rows in pivot order:
+// L unit lower below the diagonal, U upper) as X with L X = I and Y with Y U = I,
+// the block columns of X and of Y^T independent of each other: wavefronts 0
+// and 1 take X's (0 and 3, 1 and 2), 2 and 3 Y's.  For the band's pass over all
+// tiles after the factorization, in parallel and off its chain: against
+// tri_inv_lds' block products the residual of a solve is up to 20 times smaller
+// (17x13 ALEVB 7e-14 -> 1.5e-14, in FP32 5e-5 -> 2.4e-6), which saves refinement
+// sweeps and Krylov steps (17x13 ALEVB 4.67 -> 4.44 ms a step, 16 patches with FP32
+// factors 55.4 -> 50.4 ms).  Li and Ui receive full row-major tiles (zeros
+// outside the triangles, ones on L^-1's diagonal).  256 threads; rd: T entries
+// of LDS.
+template <class S>
+__device__ __forceinline__ void tri_inv_sub(S (*st)[T + 1], S *rd, S *__restrict__ Li,
+                                            S *__restrict__ Ui) {
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (threadIdx.x < T) rd[threadIdx.x] = S(1) / st[threadIdx.x][threadIdx.x];
+  __syncthreads();
+#pragma unroll 1
+  for (int h = 0; h < 2; ++h) {
+    const int J = w & 1 ? 1 + h : 3 * h;
+    if (w < 2) tri_inv_col<S, true>(J, &st[0][0], T + 1, 1, rd, Li, T, 1);
+    else tri_inv_col<S, false>(J, &st[0][0], 1, T + 1, rd, Ui, 1, T);
   }
 }
 
@@ -1354,13 +1478,13 @@ __global__ void k_span_init(unsigned long long *__restrict__ span) {
 template <class S>
 __device__ __forceinline__ void tile_inv_body(int64_t I, int tb, const S *__restrict__ band,
                                               S *__restrict__ linv, S *__restrict__ uinv) {
-  __shared__ S st[T][T + 1];
+  __shared__ S st[T][T + 1], rd[T];
   const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
   const S *D = tile_ptr(band, tb, I, I);
 #pragma unroll
   for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = D[(4 * it + w) * T + lane];
   __syncthreads();
-  tri_inv_lds<S>(st, (const int *)nullptr, linv + I * T * T, uinv + I * T * T);
+  tri_inv_sub<S>(st, rd, linv + I * T * T, uinv + I * T * T);
 }
 
 template <class S>
