@@ -389,10 +389,11 @@ void build(Ctx &c, const mafem_mesh_desc *m, const mafem_params *p) {
     }
   }
   c.band_bytes = c.band_rows() * (2 * c.tb + 1) * (int64_t)TILE * TILE * (int64_t)sizeof(double);
-  // default ordering of the single-context factorization: nested dissection
-  // where the band would be long enough to run two-ended (from about 16x16
-  // elements up), else the band; MAFEM_ORDERING=band|nd overrides
-  c.ordering = c.nt >= 8 * (int64_t)c.tb ? 1 : 0;
+  // default ordering of the single-context factorization: nested dissection on
+  // the node grid (a time step against the band's: 6x6 LAG 1.17 / 1.15 ms, 8x8
+  // LAG 1.43 / 1.29, 17x13 ALEVB 4.42 / 2.63, 24x10 LAG bending 2.97 / 2.51, 40x12
+  // EUL 7.55 / 3.00, band first); MAFEM_ORDERING=band|nd overrides
+  c.ordering = c.numnp == c.num1np * c.num2np ? 1 : 0;
   if (const char *e = std::getenv("MAFEM_ORDERING")) {
     if (std::strcmp(e, "band") == 0) c.ordering = 0;
     else if (std::strcmp(e, "nd") == 0) c.ordering = 1;

@@ -175,5 +175,57 @@ inline Plan build_plan(int64_t n1, int64_t n2, int ndf, int leaf = 4) {
   return P;
 }
 
+// What a factorization and its solve take with leaves of at most `leaf` nodes a
+// side, in microseconds.  A dependent tile step (panels, then the update with
+// the next diagonal LU) takes 33, a level's launches beside its steps
+// (assembly, Schur blocks, four of the solve) as much again, and the tile
+// products run at 45 TFLOP/s where they fill the chip.
+inline double plan_cost(int64_t n1, int64_t n2, int ndf, int leaf) {
+  std::vector<int64_t> steps;  // per level the largest fT
+  double products = 0.0;
+  std::function<size_t(int64_t, int64_t, int64_t, int64_t)> rec =
+      [&](int64_t a1, int64_t b1, int64_t a2, int64_t b2) -> size_t {
+    const int64_t w1 = b1 - a1, w2 = b2 - a2;
+    size_t lev = 0;
+    int64_t f = w1 * w2;
+    if (w1 > leaf || w2 > leaf) {
+      f = 2 * std::min(w1, w2);
+      const int64_t m = w1 >= w2 ? a1 + (w1 - 2) / 2 : a2 + (w2 - 2) / 2;
+      lev = 1 + (w1 >= w2 ? std::max(rec(a1, m, a2, b2), rec(m + 2, b1, a2, b2))
+                          : std::max(rec(a1, b1, a2, m), rec(a1, b1, m + 2, b2)));
+    }
+    // the boundary is the two lines of nodes around the box, within the grid
+    const int64_t o1 = std::min<int64_t>(2, a1) + std::min<int64_t>(2, n1 - b1);
+    const int64_t o2 = std::min<int64_t>(2, a2) + std::min<int64_t>(2, n2 - b2);
+    const int64_t b = (w1 + o1) * (w2 + o2) - w1 * w2;
+    const int64_t fT = (f * ndf + NT - 1) / NT, FT = fT + (b * ndf + NT - 1) / NT;
+    for (int64_t K = 0; K < fT; ++K) products += (double)(FT - K - 1) * (double)(FT - K);
+    if (steps.size() <= lev) steps.resize(lev + 1, 0);
+    steps[lev] = std::max(steps[lev], fT);
+    return lev;
+  };
+  rec(0, n1, 0, n2);
+  double s = (double)steps.size();
+  for (int64_t k : steps) s += (double)k;
+  return 33.0 * s + products * 2.0 * NT * NT * NT / 45e6;
+}
+
+// The leaf size of least cost.  Larger leaves save levels but lengthen the
+// leaf's own chain and cost products.  A time step with leaves of 4 and with the
+// size taken: 10x10 LAG 1.83 and 1.47 ms, 24x10 EUL 2.69 and 2.41, 96x80 LAG 11.68
+// and 11.15; 64x64 ALEVB stays at 4 (17.6 ms with 7, 16.3 with 4).
+inline int choose_leaf(int64_t n1, int64_t n2, int ndf) {
+  int best = 4;
+  double least = plan_cost(n1, n2, ndf, best);
+  for (int leaf = 5; leaf <= 10; ++leaf) {
+    const double c = plan_cost(n1, n2, ndf, leaf);
+    if (c < least) {
+      least = c;
+      best = leaf;
+    }
+  }
+  return best;
+}
+
 }  // namespace nd
 }  // namespace mafem

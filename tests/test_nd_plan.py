@@ -69,3 +69,36 @@ int main() {
     assert [int(x) for x in levels.split()] == [2, 1, 2, 2, 4, 4, 8, 8, 17]
     steps, fronts = rest.split()
     assert int(steps) == 48 and int(fronts) == 511
+
+
+def test_leaf_choice_prices_the_built_plan(tmp_path):
+    """plan_cost counts what build_plan lays out: levels, dependent steps and tile
+    products of every leaf size, on square, ragged, strip and single-front grids;
+    choose_leaf takes the least."""
+    src = r'''
+#include <cmath>
+#include <cstdio>
+#include "nd_plan.h"
+using namespace mafem::nd;
+int main() {
+  const int g[][3] = {{3, 3, 4}, {8, 8, 4}, {10, 10, 8}, {19, 15, 7}, {42, 9, 3}, {5, 60, 8}, {35, 29, 7}};
+  for (auto &x : g) {
+    double least = 1e300;
+    for (int leaf = 4; leaf <= 10; ++leaf) {
+      const Plan P = build_plan(x[0], x[1], x[2], leaf);
+      double pr = 0.0;
+      for (const Front &F : P.fr)
+        for (int K = 0; K < F.fT; ++K) pr += (double)(F.FT - K - 1) * (F.FT - K);
+      const double c = 33.0 * (P.critical_steps() + P.levels) + pr * 2 * 64 * 64 * 64 / 45e6;
+      if (std::fabs(c - plan_cost(x[0], x[1], x[2], leaf)) > 1e-9 * c) return 1;
+      least = std::fmin(least, c);
+    }
+    if (plan_cost(x[0], x[1], x[2], choose_leaf(x[0], x[1], x[2])) > least * (1 + 1e-12)) return 2;
+  }
+}
+'''
+    cpp, exe = str(tmp_path / "c.cpp"), str(tmp_path / "c")
+    with open(cpp, "w") as f:
+        f.write(src)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", CSRC, cpp, "-o", exe], check=True)
+    assert subprocess.run([exe]).returncode == 0
