@@ -247,9 +247,9 @@ int mafem_generate_output(mafem_ctx *ctx, double *xout, double *uout);
 int mafem_set_solver(mafem_ctx *ctx, const mafem_solver_opts *opts);
 
 /* Fill-reducing ordering of the context's factorization (both solver modes).
- * Default at mafem_create: MAFEM_ORDER_ND from about 16x16 elements up (where
- * the band would run two-ended), MAFEM_ORDER_BAND below; the environment
- * variable MAFEM_ORDERING=band|nd at mafem_create overrides it.
+ * Default at mafem_create: MAFEM_ORDER_ND; the environment variable
+ * MAFEM_ORDERING=band|nd at mafem_create overrides it.  Batches always factor by
+ * nested dissection.
  * MAFEM_ORDER_BAND: natural node order, band LU (two-ended on long patches),
  *   the tile rows one dependency chain.
  * MAFEM_ORDER_ND: nested dissection of the node grid (separators of two node
@@ -257,8 +257,8 @@ int mafem_set_solver(mafem_ctx *ctx, const mafem_solver_opts *opts);
  *   level of the elimination tree together, from the leaves up, each a dense
  *   tile matrix with partial pivoting inside its 64-row diagonal tiles.
  *   Fewer operations and a far shorter dependency chain than the band (64x64
- *   ALEVB: 48 dependent tile steps instead of 281), at about twice the
- *   band's factor storage.
+ *   ALEVB: 48 dependent tile steps instead of 281), at 1.2 times the band's
+ *   storage at 64x64 ALEVB, half of it at 256x256.
  * This is the role of UMFPACK's fill-reducing ordering inside `K_gl \ r_gl`
  * (src/analysis/FiniteElement.jl:38); results agree with the band's to the
  * solve tolerance, not bit for bit.  Takes effect at the next factorization. */
@@ -281,7 +281,7 @@ int mafem_device_memory(size_t *free_bytes, size_t *total_bytes);
  * step of each patch keeps the reference's definition (assembly, solve,
  * update, ε = |Δu|_2 / nmdf < εnr, at most max_iter iterations;
  * FiniteElement.jl:11-63); its linear solve is FP64 GMRES(m), right-
- * preconditioned by a band LU stored in `factor_precision` (32: the
+ * preconditioned by an LU (nested dissection) stored in `factor_precision` (32: the
  * mixed-precision path) and kept across iterations and steps; a patch is
  * refactored when a solve needs more than `refactor_iters` Arnoldi steps or
  * does not converge in `max_cycles` restart cycles, and a patch whose fresh
@@ -316,7 +316,7 @@ typedef struct {
   int64_t patch_factors;     /* sum over patches of factorizations */
   int64_t gmres_iters;       /* sum over patches of Arnoldi steps */
   int64_t elements;          /* sum over patches of area elements */
-  int32_t fp64_patches;      /* members whose band LU is stored in FP64 */
+  int32_t fp64_patches;      /* members whose LU is stored in FP64 */
   int32_t reserved;
 } mafem_batch_stats;
 

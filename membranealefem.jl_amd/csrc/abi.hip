@@ -393,7 +393,7 @@ void build(Ctx &c, const mafem_mesh_desc *m, const mafem_params *p) {
   // the node grid (a time step against the band's: 6x6 LAG 1.17 / 1.15 ms, 8x8
   // LAG 1.43 / 1.29, 17x13 ALEVB 4.42 / 2.63, 24x10 LAG bending 2.97 / 2.51, 40x12
   // EUL 7.55 / 3.00, band first); MAFEM_ORDERING=band|nd overrides
-  c.ordering = c.numnp == c.num1np * c.num2np ? 1 : 0;
+  c.ordering = 1;
   if (const char *e = std::getenv("MAFEM_ORDERING")) {
     if (std::strcmp(e, "band") == 0) c.ordering = 0;
     else if (std::strcmp(e, "nd") == 0) c.ordering = 1;

@@ -1970,243 +1970,6 @@ __global__ __launch_bounds__(SW) void k_sweep2_mw(int tb, int W, SweepChain a0, 
                          reinterpret_cast<unsigned long long *>(a.y), err);
 }
 
-// ------------------------------------------------------------ batched forms
-//
-// Patch p takes part in a factorization launch when on[p] && fac[p], and in
-// a solve launch when its flag in the given mask is set.  Factorization steps locate their patch
-// through the StepMap kernel argument; the other launches through segment
-// maps.
-
-__device__ __forceinline__ bool fac_on(const uint8_t *on, const uint8_t *fac, int p) {
-  return on[p] && fac[p];
-}
-
-// storage precision a template instance serves; patches of the other
-// precision skip the launch
-template <class S>
-constexpr int prec_of() {
-  return sizeof(S) == 4 ? 32 : 64;
-}
-
-// 64 KiB chunks of a patch's band storage, 16 bytes per store
-__global__ __launch_bounds__(256) void kb_zero_band(Seg sg, const PatchDev *__restrict__ pd,
-                                                    const uint8_t *__restrict__ on,
-                                                    const uint8_t *__restrict__ fac) {
-  const int p = sg.map[blockIdx.x];
-  if (!fac_on(on, fac, p)) return;
-  const PatchDev &d = pd[p];
-  const int64_t bytes = d.nt * (2 * d.tb + 1) * (int64_t)T * T * (d.prec / 8);
-  const int64_t base = (int64_t)(blockIdx.x - sg.blk0[p]) * 65536;
-  uint4 *dst = reinterpret_cast<uint4 *>(d.band);
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int64_t off = base + k * 4096 + threadIdx.x * 16;
-    if (off < bytes) dst[off / 16] = make_uint4(0u, 0u, 0u, 0u);
-  }
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_bsr_to_band(Seg sg, const PatchDev *__restrict__ pd,
-                                                      const uint8_t *__restrict__ on,
-                                                      const uint8_t *__restrict__ fac) {
-  const int p = sg.map[blockIdx.x];
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  bsr_to_band_body<S>(blockIdx.x - sg.blk0[p], d.nnzb, d.ndf, d.tb, d.brow, d.colidx, d.bsr,
-                      (S *)d.band);
-}
-
-// one block per patch: identity on the < 64 padding rows
-template <class S>
-__global__ __launch_bounds__(64) void kb_band_pad(const PatchDev *__restrict__ pd,
-                                                  const uint8_t *__restrict__ on,
-                                                  const uint8_t *__restrict__ fac) {
-  const int p = blockIdx.x;
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  const int64_t R = d.nx + threadIdx.x;
-  if (R < d.nt * T) tile_ptr((S *)d.band, d.tb, R / T, R / T)[(R % T) * T + (R % T)] = S(1);
-}
-
-// patch (through `order`) and block within the patch of a factorization step
-// launch; per = blocks per patch as a function of its tb
-template <int KIND>
-__device__ __forceinline__ int step_locate(const StepMap &sm, const int32_t *__restrict__ order,
-                                           int &local, int &tb) {
-  const int b = blockIdx.x;
-  int c = 0;
-  while (c + 1 < sm.ncls && b >= sm.blk0[c + 1]) ++c;
-  tb = sm.tb[c];
-  const int per = KIND == 0 ? 1 : (KIND == 1 ? 3 * tb : tb * tb);
-  const int rel = b - sm.blk0[c];
-  local = rel % per;
-  return order[sm.first[c] + rel / per];
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_diag(StepMap sm, int64_t K, const int32_t *__restrict__ order,
-                                               const PatchDev *__restrict__ pd,
-                                               const uint8_t *__restrict__ on,
-                                               const uint8_t *__restrict__ fac,
-                                               const uint8_t *__restrict__ pert) {
-  int local, tb;
-  const int p = step_locate<0>(sm, order, local, tb);
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  __shared__ __align__(16) S lds[MM_LDS];
-  if (pert[p])
-    diag_block<S, true>(K, tb, (S *)pd[p].band, pd[p].piv, pd[p].amax, lds);
-  else
-    diag_block<S, false>(K, tb, (S *)pd[p].band, pd[p].piv, nullptr, lds);
-}
-
-// max |K| of every patch of precision S that factors with static pivoting,
-// before its factorization: zeroed, then reduced over its block-sparse values
-template <class S>
-__global__ void kb_amax_zero(int P, const PatchDev *__restrict__ pd,
-                             const uint8_t *__restrict__ on, const uint8_t *__restrict__ fac,
-                             const uint8_t *__restrict__ pert) {
-  const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (p < P && fac_on(on, fac, p) && pert[p] && pd[p].prec == prec_of<S>()) pd[p].amax[0] = 0;
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_amax(Seg sg, const PatchDev *__restrict__ pd,
-                                               const uint8_t *__restrict__ on,
-                                               const uint8_t *__restrict__ fac,
-                                               const uint8_t *__restrict__ pert) {
-  const int p = sg.map[blockIdx.x];
-  if (!fac_on(on, fac, p) || !pert[p] || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  const int64_t n = d.nnzb * d.ndf * d.ndf;
-  const int64_t t = (blockIdx.x - sg.blk0[p]) * 256 + threadIdx.x;
-  double m = t < n ? fabs(d.bsr[t]) : 0.0;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0 && m > 0.0)
-    atomicMax(d.amax, (unsigned long long)__double_as_longlong(m));
-}
-
-template <class S>
-__global__ __launch_bounds__(64) void kb_panel(StepMap sm, int64_t K, const int32_t *__restrict__ order,
-                                               const PatchDev *__restrict__ pd,
-                                               const uint8_t *__restrict__ on,
-                                               const uint8_t *__restrict__ fac) {
-  int local, tb;
-  const int p = step_locate<1>(sm, order, local, tb);
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  panel_body<S>(local, K, pd[p].nt, tb, (S *)pd[p].band, pd[p].piv);
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_update(StepMap sm, int64_t K, const int32_t *__restrict__ order,
-                                                 const PatchDev *__restrict__ pd,
-                                                 const uint8_t *__restrict__ on,
-                                                 const uint8_t *__restrict__ fac) {
-  int local, tb;
-  const int p = step_locate<2>(sm, order, local, tb);
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  __shared__ __align__(16) S lds[MM_LDS];
-  update_body<S>(local, K, pd[p].nt, tb, (S *)pd[p].band, lds);
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_tile_inv(Seg sg, const PatchDev *__restrict__ pd,
-                                                  const uint8_t *__restrict__ on,
-                                                  const uint8_t *__restrict__ fac) {
-  const int p = sg.map[blockIdx.x];
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  tile_inv_body<S>(blockIdx.x - sg.blk0[p], d.tb, (const S *)d.band, (S *)d.linv, (S *)d.uinv);
-}
-
-template <class S>
-__global__ __launch_bounds__(256) void kb_fold(Seg sg, const PatchDev *__restrict__ pd,
-                                               const uint8_t *__restrict__ on,
-                                               const uint8_t *__restrict__ fac) {
-  const int p = sg.map[blockIdx.x];
-  if (!fac_on(on, fac, p) || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  __shared__ __align__(16) S lds[MM_LDS];
-  fold_body<S>(blockIdx.x - sg.blk0[p], d.nt, d.tb, (S *)d.band, (const S *)d.linv,
-               (const S *)d.uinv, lds);
-}
-
-// which = 0: t2 = L^-1 P w; which = 1: t = U^-1 t2 (per tile row)
-template <class S>
-__global__ __launch_bounds__(256) void kb_diag_apply(Seg sg, const PatchDev *__restrict__ pd,
-                                                     const uint8_t *__restrict__ mask, int which) {
-  const int p = sg.map[blockIdx.x];
-  if (!mask[p] || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  if (which == 0)
-    diag_apply_body<S>(blockIdx.x - sg.blk0[p], (const S *)d.linv, d.piv, d.w, d.t2);
-  else if (d.sweep_w > 1)  // forward result in s1 (atomic); the backward sweep reads t2
-    diag_apply_body<S>(blockIdx.x - sg.blk0[p], (const S *)d.uinv, (const int32_t *)nullptr, d.s1,
-                       d.t2, true);
-  else
-    diag_apply_body<S>(blockIdx.x - sg.blk0[p], (const S *)d.uinv, (const int32_t *)nullptr, d.t2,
-                       d.t);
-}
-
-template <class S>
-__global__ __launch_bounds__(SW) void kb_fwd_sweep(const PatchDev *__restrict__ pd,
-                                                   const uint8_t *__restrict__ mask) {
-  const int p = blockIdx.x;
-  if (!mask[p] || pd[p].prec != prec_of<S>() || pd[p].sweep_w > 1) return;
-  fwd_sweep_body<S>(pd[p].nt, pd[p].tb, (const S *)pd[p].band, pd[p].t2);
-}
-
-template <class S>
-__global__ __launch_bounds__(SW) void kb_bwd_sweep(const PatchDev *__restrict__ pd,
-                                                   const uint8_t *__restrict__ mask) {
-  const int p = blockIdx.x;
-  if (!mask[p] || pd[p].prec != prec_of<S>() || pd[p].sweep_w > 1) return;
-  bwd_sweep_body<S>(pd[p].nt, pd[p].tb, (const S *)pd[p].band, pd[p].t);
-}
-
-// Patches with sweep_w > 1 sweep over sweep_w workgroups (segment `sg`);
-// their outputs are sentinel-filled first.  which = 0: forward sweep of t2
-// into s1; which = 1: backward sweep of t2 into s2 (then collected into t).
-__global__ __launch_bounds__(256) void kb_fill_sentinel(Seg sg, const PatchDev *__restrict__ pd,
-                                                        const uint8_t *__restrict__ mask, int which,
-                                                        int prec) {
-  const int p = sg.map[blockIdx.x];
-  if (!mask[p] || pd[p].sweep_w <= 1 || pd[p].prec != prec) return;
-  const PatchDev &d = pd[p];
-  const int64_t t = (int64_t)(blockIdx.x - sg.blk0[p]) * 256 + threadIdx.x;
-  if (t < d.nt * T)
-    __hip_atomic_store(reinterpret_cast<unsigned long long *>(which == 0 ? d.s1 : d.s2) + t,
-                       SENTINEL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// t = backward-sweep output (atomic reads) for multi-workgroup patches
-__global__ __launch_bounds__(256) void kb_collect(Seg sg, const PatchDev *__restrict__ pd,
-                                                  const uint8_t *__restrict__ mask, int prec) {
-  const int p = sg.map[blockIdx.x];
-  if (!mask[p] || pd[p].sweep_w <= 1 || pd[p].prec != prec) return;
-  const PatchDev &d = pd[p];
-  const int64_t t = (int64_t)(blockIdx.x - sg.blk0[p]) * 256 + threadIdx.x;
-  if (t < d.nt * T)
-    d.t[t] = __longlong_as_double((long long)__hip_atomic_load(
-        reinterpret_cast<const unsigned long long *>(d.s2) + t, __ATOMIC_RELAXED,
-        __HIP_MEMORY_SCOPE_AGENT));
-}
-
-template <class S>
-__global__ __launch_bounds__(SW) void kb_sweep_mw(Seg sg, const PatchDev *__restrict__ pd,
-                                                  const uint8_t *__restrict__ mask, int which) {
-  const int p = sg.map[blockIdx.x];
-  if (!mask[p] || pd[p].prec != prec_of<S>()) return;
-  const PatchDev &d = pd[p];
-  const int w = (int)(blockIdx.x - sg.blk0[p]);
-  if (which == 0)
-    fwd_sweep_mw_body<S>(w, d.sweep_w, d.nt, d.tb, (const S *)d.band, d.t2,
-                         reinterpret_cast<unsigned long long *>(d.s1), d.err);
-  else
-    bwd_sweep_mw_body<S>(w, d.sweep_w, d.nt, d.tb, (const S *)d.band, d.t2,
-                         reinterpret_cast<unsigned long long *>(d.s2), d.err);
-}
-
 // ------------------------------------------------------------------ host side
 
 static inline unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -2498,7 +2261,6 @@ static void ensure_band(Ctx &c, int prec) {
   const size_t es = (prec == 32) ? sizeof(float) : sizeof(double);
   if (c.band_prec == prec && c.d_band) return;
   std::lock_guard<std::mutex> no_capture(capture_mutex());  // allocation: not during a capture
-  c.batch_factor_prec = 0;
   c.have_factor = false;
   if (c.d_band) {
     MAFEM_HIP(hipStreamSynchronize(c.stream));
@@ -2521,8 +2283,6 @@ static void ensure_band(Ctx &c, int prec) {
   c.band_bytes = (int64_t)(es * ntile);
 }
 
-void band_alloc(Ctx &c, int prec) { ensure_band(c, prec); }
-
 // nested-dissection fronts (frontal.inc, below)
 void nd_factor(Ctx &c, int prec, bool perturb);
 void nd_solve(Ctx &c, const double *rhs, double *x);
@@ -2533,7 +2293,6 @@ void band_fill(Ctx &c, int prec) {
     return;
   }
   ensure_band(c, prec);
-  c.batch_factor_prec = 0;  // the band no longer holds a batch's factorization
   if (prec == 32)
     fill_t<float>(c, (float *)c.d_band);
   else
@@ -2569,82 +2328,6 @@ void band_solve(Ctx &c, const double *d_rhs, double *d_x) {
   else
     solve_t<double>(c, (const double *)c.d_band, (const double *)c.d_linv,
                     (const double *)c.d_uinv, d_rhs, d_x);
-}
-
-template <class S>
-static void b_factor_t(BatchPlan &B, const std::vector<std::vector<StepMap>> &steps) {
-  const BatchFlags &f = B.f;
-  hipLaunchKernelGGL(kb_bsr_to_band<S>, dim3(B.bsr.nblk), dim3(256), 0, B.stream, B.bsr, B.d_pd,
-                     f.on, f.fac);
-  hipLaunchKernelGGL(kb_band_pad<S>, dim3(B.P), dim3(64), 0, B.stream, B.d_pd, f.on, f.fac);
-  hipLaunchKernelGGL(kb_amax_zero<S>, dim3((unsigned)((B.P + 255) / 256)), dim3(256), 0,
-                     B.stream, B.P, B.d_pd, f.on, f.fac, f.pert);
-  hipLaunchKernelGGL(kb_amax<S>, dim3(B.bsr.nblk), dim3(256), 0, B.stream, B.bsr, B.d_pd, f.on,
-                     f.fac, f.pert);
-  MAFEM_HIP(hipGetLastError());
-  for (int64_t K = 0; K < (int64_t)steps.size(); ++K)
-    for (const StepMap &sm : steps[K]) {
-      const int32_t nd = sm.blk0[sm.ncls];
-      StepMap smp = sm, smu = sm;
-      int32_t bp = 0, bu = 0;
-      for (int c = 0; c < sm.ncls; ++c) {
-        smp.blk0[c] = bp;
-        smu.blk0[c] = bu;
-        bp += sm.count[c] * 3 * sm.tb[c];
-        bu += sm.count[c] * sm.tb[c] * sm.tb[c];
-      }
-      smp.blk0[sm.ncls] = bp;
-      smu.blk0[sm.ncls] = bu;
-      hipLaunchKernelGGL(kb_diag<S>, dim3(nd), dim3(256), 0, B.stream, sm, K, B.d_order, B.d_pd,
-                         f.on, f.fac, f.pert);
-      hipLaunchKernelGGL(kb_panel<S>, dim3(bp), dim3(64), 0, B.stream, smp, K, B.d_order, B.d_pd,
-                         f.on, f.fac);
-      if (bu > 0)
-        hipLaunchKernelGGL(kb_update<S>, dim3(bu), dim3(256), 0, B.stream, smu, K, B.d_order,
-                           B.d_pd, f.on, f.fac);
-    }
-  hipLaunchKernelGGL(kb_tile_inv<S>, dim3(B.tiles.nblk), dim3(256), 0, B.stream, B.tiles, B.d_pd,
-                     f.on, f.fac);
-  hipLaunchKernelGGL(kb_fold<S>, dim3(B.fold.nblk), dim3(256), 0, B.stream, B.fold, B.d_pd, f.on,
-                     f.fac);
-  MAFEM_HIP(hipGetLastError());
-}
-
-void b_factor(BatchPlan &B) {
-  hipLaunchKernelGGL(kb_zero_band, dim3(B.zero.nblk), dim3(256), 0, B.stream, B.zero, B.d_pd,
-                     B.f.on, B.f.fac);
-  MAFEM_HIP(hipGetLastError());
-  if (B.has32) b_factor_t<float>(B, B.steps32);
-  if (B.has64) b_factor_t<double>(B, B.steps64);
-}
-
-template <class S>
-static void b_band_solve_t(BatchPlan &B, const uint8_t *mask) {
-  const bool mw = B.mw.nblk > 0;
-  hipLaunchKernelGGL(kb_diag_apply<S>, dim3(B.tiles.nblk), dim3(256), 0, B.stream, B.tiles, B.d_pd,
-                     mask, 0);
-  hipLaunchKernelGGL(kb_fwd_sweep<S>, dim3(B.P), dim3(SW), 0, B.stream, B.d_pd, mask);
-  if (mw) {
-    hipLaunchKernelGGL(kb_fill_sentinel, dim3(B.vec.nblk), dim3(256), 0, B.stream, B.vec, B.d_pd,
-                       mask, 0, prec_of<S>());
-    hipLaunchKernelGGL(kb_sweep_mw<S>, dim3(B.mw.nblk), dim3(SW), 0, B.stream, B.mw, B.d_pd, mask, 0);
-  }
-  hipLaunchKernelGGL(kb_diag_apply<S>, dim3(B.tiles.nblk), dim3(256), 0, B.stream, B.tiles, B.d_pd,
-                     mask, 1);
-  hipLaunchKernelGGL(kb_bwd_sweep<S>, dim3(B.P), dim3(SW), 0, B.stream, B.d_pd, mask);
-  if (mw) {
-    hipLaunchKernelGGL(kb_fill_sentinel, dim3(B.vec.nblk), dim3(256), 0, B.stream, B.vec, B.d_pd,
-                       mask, 1, prec_of<S>());
-    hipLaunchKernelGGL(kb_sweep_mw<S>, dim3(B.mw.nblk), dim3(SW), 0, B.stream, B.mw, B.d_pd, mask, 1);
-    hipLaunchKernelGGL(kb_collect, dim3(B.vec.nblk), dim3(256), 0, B.stream, B.vec, B.d_pd, mask,
-                       prec_of<S>());
-  }
-  MAFEM_HIP(hipGetLastError());
-}
-
-void b_band_solve(BatchPlan &B, const uint8_t *mask) {
-  if (B.has32) b_band_solve_t<float>(B, mask);
-  if (B.has64) b_band_solve_t<double>(B, mask);
 }
 
 }  // namespace mafem

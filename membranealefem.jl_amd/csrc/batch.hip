@@ -1,9 +1,9 @@
 // Batches: many independent patches advanced through one time step together
 // (declared in include/mafem.h).  Each member is an ordinary context; the
 // batch builds descriptors of their device buffers, the block -> patch maps
-// of every batched launch and the per-step class tables of the batched band
-// factorization, then drives the Newton iterations of all members with one
-// launch per phase.  The launch sequences are recorded once as HIP graphs
+// of every batched launch and the members' nested-dissection fronts side by
+// side, then drives the Newton iterations of all members with one launch per
+// phase (per level or tile step of the factorization and the solves).  The launch sequences are recorded once as HIP graphs
 // (assembly, factorization, refinement, update) and replayed; per-patch
 // flags in device memory decide which patches each replay touches, so the
 // graphs stay valid for every iteration and step.
@@ -33,7 +33,9 @@ struct mafem_batch {
                  g_upd = nullptr;
   std::vector<void *> owned;   // device allocations of the plan (rebuilt with it)
   std::vector<void *> fowned;  // device allocations of the flags (live with the batch)
-  std::vector<int> prec;       // band storage precision of each member
+  std::vector<int> prec;       // factor storage precision of each member
+  std::vector<const void *> store;  // where each member's factors lie
+  std::vector<uint8_t> h_fac;  // members known to be flagged for factorization
   mafem_batch_stats stats{};
 };
 
@@ -85,6 +87,8 @@ void destroy_graphs(mafem_batch &b) {
 
 void free_plan(mafem_batch &b) {
   destroy_graphs(b);
+  nd_batch_free(b.B.nd);
+  b.B.nd = nullptr;
   for (void *p : b.owned) (void)hipFree(p);
   b.owned.clear();
 }
@@ -124,83 +128,15 @@ PatchDev describe(const Ctx &c) {
   d.xms = c.d_xms; d.cps = c.d_cps; d.kel = c.d_kel; d.rel = c.d_rel;
   d.rowptr = c.d_rowptr; d.colidx = c.d_colidx; d.brow = c.d_brow; d.bsr = c.d_bsr;
   d.gptr = c.d_gptr; d.gsrc = c.d_gsrc; d.rptr = c.d_rptr; d.rsrc = c.d_rsrc;
-  d.r = c.d_r; d.b = c.d_b; d.x = c.d_x; d.w = c.d_w; d.t = c.d_t; d.t2 = c.d_t2;
-  d.band = c.d_band; d.linv = c.d_linv; d.uinv = c.d_uinv; d.piv = c.d_piv;
-  d.prec = c.band_prec;
-  d.sweep_w = 1;
-  d.s1 = c.d_s1;
-  d.s2 = c.d_s2;
-  d.err = c.d_sweep_err;
+  d.r = c.d_r; d.b = c.d_b; d.x = c.d_x; d.w = c.d_w; d.t = c.d_t;
   d.amax = c.d_amax;
   return d;
 }
 
-// Workgroups of each patch's sweeps.  A split sweep is bound by the per-row
-// hand-off (~6 us) once each workgroup streams its rows faster than that:
-// 3 workgroups for FP32 storage, 4 for FP64 are enough.  The longest chains
-// (at least 96 tile rows) get a split first, while the total stays within
-// what the device keeps resident at once (one 1024-thread sweep workgroup per
-// CU), so every workgroup a sweep waits on is running.
-void assign_sweep_groups(std::vector<PatchDev> &pd, int budget) {
-  std::vector<int> order(pd.size());
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return pd[x].nt > pd[y].nt; });
-  for (int p : order) {
-    if (pd[p].nt < 96) break;
-    const int w = pd[p].prec == 64 ? 4 : 3;
-    if (w > budget) break;
-    pd[p].sweep_w = w;
-    budget -= w;
-  }
-}
-
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Factorization step tables of the patches of one precision group.
-std::vector<std::vector<StepMap>> step_tables(const mafem_batch &b, const std::vector<int32_t> &order,
-                                              int prec) {
-  struct Cls { int first, n, tb; };
-  std::vector<Cls> cls;
-  int64_t max_nt = 0;
-  for (int i = 0; i < (int)order.size(); ++i) {
-    const PatchDev &d = b.h_pd[order[i]];
-    if (d.prec != prec) continue;
-    if (cls.empty() || cls.back().tb != d.tb || cls.back().first + cls.back().n != i)
-      cls.push_back({i, 0, d.tb});
-    cls.back().n++;
-    max_nt = std::max(max_nt, d.nt);
-  }
-  std::vector<std::vector<StepMap>> steps(max_nt);
-  for (int64_t K = 0; K < max_nt; ++K) {
-    StepMap sm{};
-    int32_t blk = 0;
-    for (const Cls &c : cls) {
-      int cnt = 0;
-      while (cnt < c.n && b.h_pd[order[c.first + cnt]].nt > K) ++cnt;
-      if (cnt == 0) continue;
-      if (sm.ncls == MAXC) {
-        sm.blk0[sm.ncls] = blk;
-        steps[K].push_back(sm);
-        sm = StepMap{};
-        blk = 0;
-      }
-      sm.first[sm.ncls] = c.first;
-      sm.count[sm.ncls] = cnt;
-      sm.tb[sm.ncls] = c.tb;
-      sm.blk0[sm.ncls] = blk;
-      blk += cnt;
-      sm.ncls++;
-    }
-    if (sm.ncls > 0) {
-      sm.blk0[sm.ncls] = blk;
-      steps[K].push_back(sm);
-    }
-  }
-  return steps;
-}
-
-// Builds descriptors, segment maps and factorization step tables (the flags
-// are allocated once per batch and keep their contents).
+// Builds descriptors, segment maps and the members' fronts (the flags are
+// allocated once per batch and keep their contents).
 void build_plan(mafem_batch &b) {
   free_plan(b);
   BatchPlan &B = b.B;
@@ -211,19 +147,21 @@ void build_plan(mafem_batch &b) {
   B.escalate_iters = b.opts.escalate_iters;
   B.rtol = b.opts.rtol;
   b.h_pd.resize(P);
-  B.has32 = B.has64 = false;
-  for (int p = 0; p < P; ++p) {
-    Ctx &c = b.members[p]->c;
-    band_alloc(c, b.prec[p]);
-    b.h_pd[p] = describe(c);
-    b.h_pd[p].V = balloc<double>(b, (B.m + 1) * c.nt * (int64_t)TILE);
-    (b.prec[p] == 32 ? B.has32 : B.has64) = true;
+  std::vector<Ctx *> ctx(P);
+  for (int p = 0; p < P; ++p) ctx[p] = &b.members[p]->c;
+  try {
+    B.nd = nd_batch_create(ctx.data(), b.prec.data(), P);
+  } catch (const ArgError &e) {
+    throw BatchError{"batch: " + e.msg, e.code};
   }
-  int dev_cus = 0;
-  MAFEM_HIP(hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, b.dev));
-  int mw_budget = (3 * dev_cus) / 4;
-  if (const char *e = std::getenv("MAFEM_BATCH_SWEEP_BUDGET")) mw_budget = std::atoi(e);
-  assign_sweep_groups(b.h_pd, mw_budget);
+  b.store.resize(P);
+  for (int p = 0; p < P; ++p) {
+    const Ctx &c = *ctx[p];
+    b.store[p] = nd_store(c);
+    b.h_pd[p] = describe(c);
+    b.h_pd[p].prec = b.prec[p];
+    b.h_pd[p].V = balloc<double>(b, (B.m + 1) * c.nt * (int64_t)TILE);
+  }
   B.d_pd = bupload(b, b.h_pd);
 
   // segment maps
@@ -244,40 +182,16 @@ void build_plan(mafem_batch &b) {
     B.area.push_back(make_seg(b, ba, 256));
     B.edge.push_back(make_seg(b, be, 256));
   }
-  std::vector<int64_t> bb(P), bv(P), bn(P), bz(P), bt(P), bf(P);
+  std::vector<int64_t> bb(P), bv(P), bn(P);
   for (int p = 0; p < P; ++p) {
     const PatchDev &d = b.h_pd[p];
     bb[p] = cdiv(d.nnzb * d.ndf * d.ndf, 256);
     bv[p] = cdiv(d.nt * TILE, 256);
     bn[p] = cdiv(d.numnp, 256);
-    bz[p] = cdiv(d.nt * (2 * d.tb + 1) * (int64_t)TILE * TILE * (d.prec / 8), 65536);
-    bt[p] = d.nt;
-    bf[p] = d.nt * (2 * d.tb + 1);
   }
   B.bsr = make_seg(b, bb, 256);
   B.vec = make_seg(b, bv, 256);
   B.node = make_seg(b, bn, 256);
-  B.zero = make_seg(b, bz, 256);
-  B.tiles = make_seg(b, bt, 256);  // tile inversion, diagonal products
-  B.fold = make_seg(b, bf, 256);
-  std::vector<int64_t> bw(P);
-  for (int p = 0; p < P; ++p) bw[p] = b.h_pd[p].sweep_w > 1 ? b.h_pd[p].sweep_w : 0;
-  B.mw = make_seg(b, bw, 1024);  // multi-workgroup sweeps
-
-  // factorization order: by precision, then classes of equal tb, each by
-  // decreasing nt
-  std::vector<int32_t> order(P);
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
-    const PatchDev &a = b.h_pd[x], &c = b.h_pd[y];
-    if (a.prec != c.prec) return a.prec < c.prec;
-    return a.tb != c.tb ? a.tb < c.tb : a.nt > c.nt;
-  });
-  B.d_order = bupload(b, order);
-  B.steps32 = step_tables(b, order, 32);
-  B.steps64 = step_tables(b, order, 64);
-  B.max_nt = 0;
-  for (const PatchDev &d : b.h_pd) B.max_nt = std::max(B.max_nt, d.nt);
   B.f.part = balloc<double>(b, std::max<int64_t>(B.vec.nblk, 1));
   B.f.part2 = balloc<double>(b, std::max<int64_t>((int64_t)B.vec.nblk * (B.m + 1), 1));
 }
@@ -331,12 +245,12 @@ void ensure_hist(mafem_batch &b, int max_iter) {
   B.f.eps_hist = falloc<double>(b, (int64_t)B.P * max_iter);
 }
 
-// The plan is stale when a member's band storage moved (a precision change
+// The plan is stale when a member's factor storage moved (a precision change
 // through its own solver entry points).
 bool plan_stale(const mafem_batch &b) {
   for (size_t p = 0; p < b.members.size(); ++p) {
     const Ctx &c = b.members[p]->c;
-    if (c.d_band != b.h_pd[p].band || c.band_prec != b.prec[p]) return true;
+    if (nd_store(c) != b.store[p] || nd_prec(c) != b.prec[p]) return true;
   }
   return false;
 }
@@ -386,7 +300,7 @@ void run(mafem_batch &b, hipGraphExec_t &g, void (*issue)(mafem_batch &)) {
 }
 
 // Patches whose fresh FP32 factorization could not precondition the solve
-// move to FP64 band storage: the plan is rebuilt around them (flags and
+// move to FP64 factors: the plan is rebuilt around them (flags and
 // iterates are kept) and they are refactored before the solve continues.
 void escalate(mafem_batch &b) {
   const int P = b.B.P;
@@ -478,7 +392,7 @@ int mafem_batch_create(mafem_batch **out, int32_t n, mafem_ctx *const *members,
       for (auto &e : b.ev) MAFEM_HIP(hipEventCreate(&e));
       MAFEM_HIP(hipHostMalloc((void **)&b.h_count, 32, hipHostMallocDefault));
       // a member keeps the precision a previous batch chose for it and, when
-      // still valid, the factorization that batch left in its band
+      // still valid, the factorization that batch left in its fronts
       b.prec.resize(n);
       for (int32_t i = 0; i < n; ++i) {
         const Ctx &c = members[i]->c;
@@ -489,8 +403,9 @@ int mafem_batch_create(mafem_batch **out, int32_t n, mafem_ctx *const *members,
       std::vector<uint8_t> fac(n);
       for (int32_t i = 0; i < n; ++i) {
         const Ctx &c = members[i]->c;
-        fac[i] = (c.batch_factor_prec == b.prec[i] && c.band_prec == b.prec[i]) ? 0 : 1;
+        fac[i] = (c.batch_factor_prec == b.prec[i] && nd_prec(c) == b.prec[i]) ? 0 : 1;
       }
+      b.h_fac = fac;
       MAFEM_HIP(hipMemcpy(b.B.f.fac, fac.data(), n, hipMemcpyHostToDevice));
     } catch (const HipError &h) {
       b.err = std::string("HIP error ") + hipGetErrorString(h.code) + " in " + h.what;
@@ -546,13 +461,19 @@ int mafem_batch_time_step(mafem_batch *bp, const double *time, const double *dt,
     const int P = B.P;
     for (mafem_ctx *m : b.members) {
       MAFEM_HIP(hipStreamSynchronize(m->c.stream));
-      // the batch factors into the member's band in its own (one-chain) layout:
-      // a factorization the context kept for its own Krylov solves is gone
+      // the batch factors into the member's fronts: a factorization the context
+      // kept there for its own Krylov solves is gone
       m->c.have_factor = false;
     }
     if (plan_stale(b)) build_plan(b);
     ensure_hist(b, max_iter);
     BatchFlags &f = B.f;
+    // and a member that has factored for itself since is factored afresh
+    const uint8_t one = 1;
+    for (int p = 0; p < P; ++p)
+      if (b.members[p]->c.batch_factor_prec != b.prec[p] && !b.h_fac[p])
+        MAFEM_HIP(hipMemcpyAsync(f.fac + p, &one, 1, hipMemcpyHostToDevice, B.stream));
+    std::fill(b.h_fac.begin(), b.h_fac.end(), 0);
     std::vector<uint8_t> ones8(P, 1);
     if (active)
       for (int p = 0; p < P; ++p) ones8[p] = active[p] ? 1 : 0;
@@ -668,20 +589,8 @@ int mafem_batch_time_step(mafem_batch *bp, const double *time, const double *dt,
         for (int k = 0; k < max_iter; ++k)
           eps_hist[(size_t)p * max_iter + k] = k < h_it[p] ? h_hist[(size_t)p * max_iter + k] : 0.0;
     }
-    // multi-workgroup sweeps whose waits ran out invalidate the step
-    for (int p = 0; p < P; ++p) {
-      if (b.h_pd[p].sweep_w <= 1) continue;
-      int e = 0;
-      MAFEM_HIP(hipMemcpy(&e, b.h_pd[p].err, sizeof(int), hipMemcpyDeviceToHost));
-      if (e != 0) {
-        MAFEM_HIP(hipMemset(b.h_pd[p].err, 0, sizeof(int)));
-        throw BatchError{"a triangular sweep wait ran out: this step's corrections are invalid "
-                         "and so are the member states they updated (set them again "
-                         "before continuing)", MAFEM_EHIP};
-      }
-    }
-    // what each member's band holds now, for a later batch
-    std::vector<uint8_t> h_fac(P);
+    // what each member's fronts hold now, for a later batch
+    std::vector<uint8_t> &h_fac = b.h_fac;
     MAFEM_HIP(hipMemcpy(h_fac.data(), f.fac, P, hipMemcpyDeviceToHost));
     for (int p = 0; p < P; ++p) {
       Ctx &c = b.members[p]->c;

@@ -49,7 +49,8 @@ struct EdgeItem {
   double nval;
 };
 
-struct NdDev;  // nested-dissection fronts (band.hip)
+struct NdDev;    // nested-dissection fronts (band.hip)
+struct NdBatch;  // those of a batch's members
 
 struct Ctx {
   std::string err;
@@ -136,7 +137,7 @@ struct Ctx {
   mafem_stats stats{};
   int32_t n_band_solve = 0;     // running count of triangular-solve sweeps
 
-  // factorization left in the band by a batch (kept when the context joins
+  // factorization left in the fronts by a batch (kept when the context joins
   // another batch): its precision, 0 = none; batch_prec = precision a batch
   // last chose for this context (an FP64 fallback stays FP64)
   int batch_factor_prec = 0;
@@ -231,14 +232,9 @@ struct PatchDev {
   const int32_t *rowptr, *colidx, *brow;
   double *bsr;
   const int64_t *gptr, *gsrc, *rptr, *rsrc;
-  double *r, *b, *x, *w, *t, *t2;
-  void *band, *linv, *uinv;
-  int32_t *piv;
+  double *r, *b, *x, *w, *t;
   double *V;         // GMRES basis, m + 1 vectors of length nt TILE (batch-owned)
-  int32_t prec;      // band storage precision of this patch: 32 or 64
-  int32_t sweep_w;   // workgroups of its triangular sweeps
-  double *s1, *s2;   // forward/backward outputs of multi-workgroup sweeps (atomic access only)
-  int *err;          // count of sweep waits that ran out
+  int32_t prec;      // factor storage precision of this patch: 32 or 64
   unsigned long long *amax;  // static pivoting: max |K| bits, replaced-pivot count
 };
 
@@ -247,19 +243,6 @@ struct Seg {
   int32_t *map = nullptr;   // [nblk] patch of each block
   int64_t *blk0 = nullptr;  // [P] first block of each patch (unused patches: -1)
   unsigned nblk = 0;
-};
-
-// Patches active at one step K of the batched factorization, grouped in
-// classes of equal tile half-bandwidth; patches are listed in `order`
-// (class by class, each class by decreasing tile-row count), so the active
-// members of a class are a prefix of it.
-constexpr int MAXC = 40;
-struct StepMap {
-  int32_t ncls;
-  int32_t first[MAXC];   // index into order of the class's first patch
-  int32_t count[MAXC];   // active patches of the class at this step
-  int32_t tb[MAXC];
-  int32_t blk0[MAXC + 1];  // first block of the class in this launch
 };
 
 // Per-patch flags and scalars of a batch, all in device memory.  The linear
@@ -295,7 +278,6 @@ struct BatchFlags {
 
 struct BatchPlan {
   int P = 0;
-  bool has32 = false, has64 = false;  // precision groups present
   int max_iter = 14;
   int m = 20;                // GMRES basis size
   int refactor_iters = 6;
@@ -303,28 +285,29 @@ struct BatchPlan {
   double rtol = 1e-10;
   hipStream_t stream = nullptr;
   PatchDev *d_pd = nullptr;
-  int32_t *d_order = nullptr;
+  NdBatch *nd = nullptr;            // the members' fronts and their launches
   BatchFlags f{};
   std::vector<int> motions;         // motions present
   std::vector<Seg> area, edge;      // per motion present
-  Seg bsr, vec, node, zero, tiles, fold;
-  Seg mw;                           // blocks of the multi-workgroup sweeps
-  std::vector<std::vector<StepMap>> steps32, steps64;  // factorization steps per precision group
-  int64_t max_nt = 0;
+  Seg bsr, vec, node;
 };
 
 // batched launch sequences (assemble.hip, band.hip, vec.hip)
 void b_assemble(BatchPlan &B);
 void b_predict(BatchPlan &B);
 void b_factor(BatchPlan &B);
-void b_band_solve(BatchPlan &B, const uint8_t *mask);  // t = LU^-1 w where mask
+void b_lu_solve(BatchPlan &B, const uint8_t *mask);  // t = LU^-1 w where mask
 void b_solve_begin(BatchPlan &B);  // sol = on; b = -r, x = 0, |b|, kits = 0
 void b_gmres_cycle(BatchPlan &B);  // one restart cycle for patches with sol
 void b_solve_end(BatchPlan &B);    // unconverged solves: refactor and redo, or give up
 void b_update(BatchPlan &B);       // refactor policy, state update, ε, Newton flags, counts
 void b_mark_factored(BatchPlan &B);
 void b_count(BatchPlan &B);        // count[0] = on, count[2] = on && fac
-void band_alloc(Ctx &c, int prec); // band storage of the given precision
+// fronts of every member in the given precisions, side by side; nd_store: where a
+// context's factors lie (null: nowhere yet)
+NdBatch *nd_batch_create(Ctx *const *members, const int *prec, int n);
+void nd_batch_free(NdBatch *B);
+const void *nd_store(const Ctx &c);
 
 // Serialises graph recording against context creation on other host threads
 // (creation makes synchronous null-stream copies, which would invalidate a

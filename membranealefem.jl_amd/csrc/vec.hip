@@ -516,9 +516,12 @@ __global__ __launch_bounds__(256) void kb_add_t(Seg sg, const PatchDev *__restri
   if (at.t < d.nt * TILE) d.x[at.t] += d.t[at.t];
 }
 
-// after a cycle: the true relative residual decides; converged solves leave sol
+// after a cycle: the true relative residual decides; converged solves leave sol,
+// and where the factors were singular (an infinite or undefined residual) the
+// next attempt starts from zero again
 __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__restrict__ pd,
                                                     BatchFlags f, double rtol) {
+  __shared__ int bad;
   const int p = blockIdx.x;
   if (!f.sol[p]) return;
   const double s = patch_sum(sg, f.part, p, vec_blocks(pd[p]));
@@ -526,7 +529,11 @@ __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__re
     const double rr = sqrt(s) / f.bn[p];
     f.relres[p] = rr;
     if (rr <= rtol) f.sol[p] = 0;
+    bad = isfinite(rr) ? 0 : 1;
   }
+  __syncthreads();
+  if (bad)
+    for (int64_t t = threadIdx.x; t < pd[p].nt * TILE; t += 256) pd[p].x[t] = 0.0;
 }
 
 // count[1] = solves still unconverged
@@ -717,7 +724,7 @@ void b_gmres_cycle(BatchPlan &B) {
   hipLaunchKernelGGL(kb_set_v, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon, f.scale, 0);
   for (int j = 0; j < B.m; ++j) {
     hipLaunchKernelGGL(kb_get_v, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon, j);
-    b_band_solve(B, f.kon);
+    b_lu_solve(B, f.kon);
     hipLaunchKernelGGL(kb_spmv_t, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon);
     for (int pass = 0; pass < 2; ++pass) {  // classical Gram-Schmidt, twice
       hipLaunchKernelGGL(kb_mdot, dim3(nv, j + 1), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon,
@@ -736,7 +743,7 @@ void b_gmres_cycle(BatchPlan &B) {
   }
   hipLaunchKernelGGL(kb_ysolve, dim3((B.P + 63) / 64), dim3(64), 0, B.stream, B.P, f, B.m);
   hipLaunchKernelGGL(kb_vcomb, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.m);
-  b_band_solve(B, f.sol);
+  b_lu_solve(B, f.sol);
   hipLaunchKernelGGL(kb_add_t, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol);
   hipLaunchKernelGGL(kb_resid, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol, f.part);
   hipLaunchKernelGGL(kb_cycle_end, dim3(B.P), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.rtol);

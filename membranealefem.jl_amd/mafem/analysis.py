@@ -214,8 +214,8 @@ class Batch:
 
     No counterpart in the reference (one mesh per `solve`); each member's
     Newton step keeps the reference's definition (FiniteElement.jl:11-63).
-    The linear solves run as FP64 GMRES(restart) right-preconditioned by a
-    band LU kept in `precision` (32: mixed precision).  The members are
+    The linear solves run as FP64 GMRES(restart) right-preconditioned by an
+    LU kept in `precision` (32: mixed precision).  The members are
     borrowed: keep them alive while the batch exists.
     """
 

@@ -112,9 +112,10 @@ class Patch:
 
 def device_bytes(spec: PatchSpec, precision=32, restart=20, ordering="band"):
     """Device memory of one patch context plus its batch storage (bytes).
-    ordering "nd": its factorization held as nested-dissection fronts instead
-    of a band, bounded by five times the FP64 band (fronts of 32x32 to 128x128
-    patches measure 4.9 to 2.7 times it)."""
+    ordering "nd": its factorization held as nested-dissection fronts (as batches
+    do) instead of a band, bounded by 2.5 times the one-chain band of the same
+    precision and less from 45 nodes a side on (fronts of 16x16, 40x40, 66x66 and
+    96x96 patches measure at most 2.25, 1.75, 1.6 and 1.05 times it)."""
     ndf = {int(LAG): 4, int(EUL): 7}.get(int(spec.motion), 8)
     n = spec.n
     numel = n * n
@@ -128,7 +129,7 @@ def device_bytes(spec: PatchSpec, precision=32, restart=20, ordering="band"):
     rows = nt + tb if nt >= 8 * tb else nt  # the two-ended layout keeps tb more tile rows
     band = rows * (2 * tb + 1) * 64 * 64 * es + 2 * rows * 64 * 64 * es
     if ordering == "nd":
-        band = 5 * (rows * (2 * tb + 1) * 64 * 64 * 8 + 2 * rows * 64 * 64 * 8)
+        band = int(min(2.5, max(1.1, 112 / n1)) * nt * (2 * tb + 3) * 64 * 64 * es)
     nnzb = numnp * 25
     kel = (numel + 4 * n) * ne * ne * 8
     bsr = nnzb * ndf * ndf * 8

@@ -91,10 +91,8 @@ class Server:
         self.solo_count = 0
 
     def _bytes(self, r):
-        # FP64 band storage in the estimate (a member may fall back to it);
-        # requests large enough to run solo factor with nested dissection
-        solo = r.spec.n * r.spec.n >= self.solo_min_elements
-        return int(1.15 * device_bytes(r.spec, precision=64, ordering="nd" if solo else "band"))
+        # FP64 storage in the estimate (a member may fall back to it)
+        return int(1.15 * device_bytes(r.spec, precision=64, ordering="nd"))
 
     def run(self, requests, time_limit=None, log=None):
         """Serve `requests` (sorted by arrival); returns them with results."""

@@ -102,3 +102,40 @@ int main() {
         f.write(src)
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", CSRC, cpp, "-o", exe], check=True)
     assert subprocess.run([exe]).returncode == 0
+
+
+def test_schur_complements_that_coexist_do_not_overlap(tmp_path):
+    """place_schur: complements that are there on a common level (from their
+    front's to its parent's) lie apart, inside the pool, and the pool is smaller
+    than all of them once a tree has a few levels."""
+    src = r'''
+#include <cstdio>
+#include "nd_plan.h"
+using namespace mafem::nd;
+int main() {
+  const int g[][4] = {{3, 3, 4, 4}, {6, 5, 8, 4}, {8, 8, 4, 4}, {19, 15, 7, 4}, {42, 9, 3, 5}, {5, 60, 8, 4}, {35, 29, 7, 6}};
+  for (auto &x : g) {
+    const Plan P = build_plan(x[0], x[1], x[2], x[3]);
+    std::vector<int64_t> at;
+    const int64_t total = place_schur(P, at);
+    int64_t sum = 0;
+    auto size = [&](size_t t) { return (int64_t)(P.fr[t].FT - P.fr[t].fT) * (P.fr[t].FT - P.fr[t].fT); };
+    for (size_t t = 0; t < P.fr.size(); ++t) {
+      if (P.fr[t].parent < 0) continue;
+      sum += size(t);
+      if (at[t] < 0 || at[t] + size(t) > total) return 1;
+      for (size_t u = 0; u < t; ++u) {
+        if (P.fr[u].parent < 0) continue;
+        const bool meet = P.fr[t].level <= P.fr[P.fr[u].parent].level && P.fr[u].level <= P.fr[P.fr[t].parent].level;
+        if (meet && at[t] < at[u] + size(u) && at[u] < at[t] + size(t)) return 2;
+      }
+    }
+    if (P.levels > 4 && total >= sum) return 3;
+  }
+}
+'''
+    cpp, exe = str(tmp_path / "c.cpp"), str(tmp_path / "c")
+    with open(cpp, "w") as f:
+        f.write(src)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", CSRC, cpp, "-o", exe], check=True)
+    assert subprocess.run([exe]).returncode == 0
