@@ -29,8 +29,9 @@ struct mafem_batch {
   int dev = 0;
   hipEvent_t ev[8] = {};
   int32_t *h_count = nullptr;  // pinned mirror of B.f.count
-  hipGraphExec_t g_asm = nullptr, g_fac = nullptr, g_cyc = nullptr, g_end = nullptr,
+  hipGraphExec_t g_asm = nullptr, g_fac = nullptr, g_fin = nullptr, g_end = nullptr,
                  g_upd = nullptr;
+  std::vector<hipGraphExec_t> g_arn;  // chunks of a cycle's Arnoldi steps
   std::vector<void *> owned;   // device allocations of the plan (rebuilt with it)
   std::vector<void *> fowned;  // device allocations of the flags (live with the batch)
   std::vector<int> prec;       // factor storage precision of each member
@@ -78,11 +79,14 @@ T *bupload(mafem_batch &b, const std::vector<T> &v) {
 }
 
 void destroy_graphs(mafem_batch &b) {
-  for (hipGraphExec_t *g : {&b.g_asm, &b.g_fac, &b.g_cyc, &b.g_end, &b.g_upd})
+  for (hipGraphExec_t *g : {&b.g_asm, &b.g_fac, &b.g_fin, &b.g_end, &b.g_upd})
     if (*g) {
       (void)hipGraphExecDestroy(*g);
       *g = nullptr;
     }
+  for (hipGraphExec_t g : b.g_arn)
+    if (g) (void)hipGraphExecDestroy(g);
+  b.g_arn.clear();
 }
 
 void free_plan(mafem_batch &b) {
@@ -286,17 +290,41 @@ void issue_fac(mafem_batch &b) {
   b_factor(b.B);
   b_mark_factored(b.B);
 }
-void issue_cyc(mafem_batch &b) { b_gmres_cycle(b.B); }
+void issue_fin(mafem_batch &b) { b_cycle_end(b.B); }
 void issue_end(mafem_batch &b) { b_solve_end(b.B); }
 void issue_upd(mafem_batch &b) { b_update(b.B); }
 
-void run(mafem_batch &b, hipGraphExec_t &g, void (*issue)(mafem_batch &)) {
+template <class F>
+void run(mafem_batch &b, hipGraphExec_t &g, F &&issue) {
   if (!b.opts.use_graphs) {
     issue(b);
     return;
   }
   if (!g) g = record(b, [&] { issue(b); });
   MAFEM_HIP(hipGraphLaunch(g, b.B.stream));
+}
+
+void read_counts(mafem_batch &b);
+
+// Arnoldi steps between two looks at who goes on.  A step is some 40 launches
+// (130 us at 16 patches of 16 to 40 a side, as much when no patch is in it any
+// more), a look 25 us; solves take 3 to 6 steps of the 20 a cycle may have.
+constexpr int ARNOLDI_CHUNK = 2;
+
+// One restart cycle, ended when no patch goes on.
+void run_cycle(mafem_batch &b) {
+  const int m = b.B.m, n = (m + ARNOLDI_CHUNK - 1) / ARNOLDI_CHUNK;
+  b.g_arn.resize(n, nullptr);
+  for (int k = 0; k < n; ++k) {
+    run(b, b.g_arn[k], [k, m](mafem_batch &q) {
+      if (k == 0) b_cycle_begin(q.B);
+      b_cycle_steps(q.B, k * ARNOLDI_CHUNK, std::min(m, (k + 1) * ARNOLDI_CHUNK));
+    });
+    if (k + 1 == n) break;
+    read_counts(b);
+    if (b.h_count[5] == 0) break;
+  }
+  run(b, b.g_fin, issue_fin);
 }
 
 // Patches whose fresh FP32 factorization could not precondition the solve
@@ -517,7 +545,7 @@ int mafem_batch_time_step(mafem_batch *bp, const double *time, const double *dt,
         }
         for (int cyc = 0; cyc < b.opts.max_cycles; ++cyc) {
           MAFEM_HIP(hipEventRecord(b.ev[5], B.stream));
-          run(b, b.g_cyc, issue_cyc);
+          run_cycle(b);
           MAFEM_HIP(hipEventRecord(b.ev[6], B.stream));
           ++st.gmres_cycles;
           read_counts(b);

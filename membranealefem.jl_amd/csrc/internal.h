@@ -298,7 +298,11 @@ void b_predict(BatchPlan &B);
 void b_factor(BatchPlan &B);
 void b_lu_solve(BatchPlan &B, const uint8_t *mask);  // t = LU^-1 w where mask
 void b_solve_begin(BatchPlan &B);  // sol = on; b = -r, x = 0, |b|, kits = 0
-void b_gmres_cycle(BatchPlan &B);  // one restart cycle for patches with sol
+// one restart cycle for patches with sol: its start, Arnoldi steps j0 .. j1 - 1
+// (count[5] = patches that go on after them) and its end
+void b_cycle_begin(BatchPlan &B);
+void b_cycle_steps(BatchPlan &B, int j0, int j1);
+void b_cycle_end(BatchPlan &B);
 void b_solve_end(BatchPlan &B);    // unconverged solves: refactor and redo, or give up
 void b_update(BatchPlan &B);       // refactor policy, state update, ε, Newton flags, counts
 void b_mark_factored(BatchPlan &B);

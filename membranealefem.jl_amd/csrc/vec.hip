@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256) void kb_cycle_start(Seg sg, const PatchDev *__
   }
 }
 
-// V_j = scale w
+// V_j = scale w, and w = V_j (input of the preconditioner)
 __global__ __launch_bounds__(256) void kb_set_v(Seg sg, const PatchDev *__restrict__ pd,
                                                 const uint8_t *__restrict__ mask,
                                                 const double *__restrict__ scale, int j) {
@@ -355,17 +355,7 @@ __global__ __launch_bounds__(256) void kb_set_v(Seg sg, const PatchDev *__restri
   if (!mask[at.p]) return;
   const PatchDev &d = pd[at.p];
   const int64_t ld = d.nt * TILE;
-  if (at.t < ld) d.V[j * ld + at.t] = scale[at.p] * d.w[at.t];
-}
-
-// w = V_j (input of the preconditioner)
-__global__ __launch_bounds__(256) void kb_get_v(Seg sg, const PatchDev *__restrict__ pd,
-                                                const uint8_t *__restrict__ mask, int j) {
-  const VecAt at = vec_at(sg);
-  if (!mask[at.p]) return;
-  const PatchDev &d = pd[at.p];
-  const int64_t ld = d.nt * TILE;
-  if (at.t < ld) d.w[at.t] = d.V[j * ld + at.t];
+  if (at.t < ld) d.V[j * ld + at.t] = d.w[at.t] = scale[at.p] * d.w[at.t];
 }
 
 // w = K t (padding rows: 0)
@@ -534,6 +524,14 @@ __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__re
   __syncthreads();
   if (bad)
     for (int64_t t = threadIdx.x; t < pd[p].nt * TILE; t += 256) pd[p].x[t] = 0.0;
+}
+
+// count[5] = Arnoldi processes still running
+__global__ __launch_bounds__(256) void kb_count_kon(int P, BatchFlags f) {
+  int n = 0;
+  for (int p = threadIdx.x; p < P; p += 256) n += f.kon[p];
+  const double r = block_sum((double)n);
+  if (threadIdx.x == 0) f.count[5] = (int32_t)r;
 }
 
 // count[1] = solves still unconverged
@@ -715,15 +713,20 @@ void b_solve_begin(BatchPlan &B) {
   MAFEM_HIP(hipGetLastError());
 }
 
-void b_gmres_cycle(BatchPlan &B) {
+void b_cycle_begin(BatchPlan &B) {
   const BatchFlags &f = B.f;
   const unsigned nv = B.vec.nblk;
   hipLaunchKernelGGL(kb_resid, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol, f.part);
   hipLaunchKernelGGL(kb_cycle_start, dim3(B.P), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.m,
                      B.rtol);
   hipLaunchKernelGGL(kb_set_v, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon, f.scale, 0);
-  for (int j = 0; j < B.m; ++j) {
-    hipLaunchKernelGGL(kb_get_v, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon, j);
+  MAFEM_HIP(hipGetLastError());
+}
+
+void b_cycle_steps(BatchPlan &B, int j0, int j1) {
+  const BatchFlags &f = B.f;
+  const unsigned nv = B.vec.nblk;
+  for (int j = j0; j < j1; ++j) {
     b_lu_solve(B, f.kon);
     hipLaunchKernelGGL(kb_spmv_t, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon);
     for (int pass = 0; pass < 2; ++pass) {  // classical Gram-Schmidt, twice
@@ -741,6 +744,13 @@ void b_gmres_cycle(BatchPlan &B) {
                          j + 1);
     MAFEM_HIP(hipGetLastError());
   }
+  hipLaunchKernelGGL(kb_count_kon, dim3(1), dim3(256), 0, B.stream, B.P, f);
+  MAFEM_HIP(hipGetLastError());
+}
+
+void b_cycle_end(BatchPlan &B) {
+  const BatchFlags &f = B.f;
+  const unsigned nv = B.vec.nblk;
   hipLaunchKernelGGL(kb_ysolve, dim3((B.P + 63) / 64), dim3(64), 0, B.stream, B.P, f, B.m);
   hipLaunchKernelGGL(kb_vcomb, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.m);
   b_lu_solve(B, f.sol);
