@@ -58,7 +58,7 @@ void free_all(Ctx &c) {
     if (p) (void)hipFree(p);
   nd_free(c);
   if (c.h_red) (void)hipHostFree(c.h_red);
-  for (auto &e : c.ev)
+  for (auto &e : c.evs)
     if (e) (void)hipEventDestroy(e);
   if (c.stream) (void)hipStreamDestroy(c.stream);
 }
@@ -84,14 +84,6 @@ namespace {
 int fail(Ctx &c, const std::string &m, int code) {
   c.err = m;
   return code;
-}
-
-// running count of replaced pivots (blocking read of the device counter)
-int32_t read_pert(Ctx &c) {
-  unsigned long long v[2] = {0, 0};
-  MAFEM_HIP(hipMemcpyAsync(v, c.d_amax, sizeof(v), hipMemcpyDeviceToHost, c.stream));
-  MAFEM_HIP(hipStreamSynchronize(c.stream));
-  return (int32_t)v[1];
 }
 
 int from_hip(Ctx &c, const HipError &h) {
@@ -401,7 +393,7 @@ void build(Ctx &c, const mafem_mesh_desc *m, const mafem_params *p) {
 
   // device allocations and uploads
   MAFEM_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-  for (auto &e : c.ev) MAFEM_HIP(hipEventCreate(&e));
+  for (auto &e : c.evs) MAFEM_HIP(hipEventCreate(&e));
   c.d_xms = dalloc<double>(c, numnp * 3);
   c.d_cps = dalloc<double>(c, numnp * ndf);
   MAFEM_HIP(hipMemset(c.d_xms, 0, sizeof(double) * numnp * 3));
@@ -432,8 +424,9 @@ void build(Ctx &c, const mafem_mesh_desc *m, const mafem_params *p) {
   c.d_t2 = dalloc<double>(c, nv);
   for (double *v : {c.d_r, c.d_x, c.d_w, c.d_t, c.d_b, c.d_t2})
     MAFEM_HIP(hipMemset(v, 0, sizeof(double) * nv));
-  c.d_red = dalloc<double>(c, 512);
-  MAFEM_HIP(hipHostMalloc((void **)&c.h_red, sizeof(double) * 16, hipHostMallocDefault));
+  c.d_red = dalloc<double>(c, 3 * NRED + 8);
+  MAFEM_HIP(hipMemset(c.d_red + 3 * NRED, 0, sizeof(double) * 8));
+  MAFEM_HIP(hipHostMalloc((void **)&c.h_red, sizeof(double) * RED_N, hipHostMallocDefault));
   c.d_eq = dupload(c, eq_ext);
   c.opts = mafem_solver_opts{MAFEM_SOLVER_DIRECT, 64, 30, 200, 20, 3, 1e-13};
   c.d_piv = dalloc<int32_t>(c, c.band_rows() * TILE);
@@ -535,11 +528,21 @@ __global__ void k_scatter_idx(int64_t n, const int64_t *__restrict__ idx,
 
 inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-float elapsed(Ctx &c, int a, int b) {
+float elapsed(const hipEvent_t *ev, int a, int b) {
   float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, c.ev[a], c.ev[b]);
+  (void)hipEventElapsedTime(&ms, ev[a], ev[b]);
   return ms;
 }
+float elapsed(Ctx &c, int a, int b) { return elapsed(c.ev, a, b); }
+
+// static pivoting's count of replaced pivots and the count of waits that ran out,
+// into pinned host memory at the end of a time step
+__global__ void k_step_end(const unsigned long long *__restrict__ amax, const int *__restrict__ err,
+                           double *__restrict__ out) {
+  out[0] = (double)amax[1];
+  out[1] = (double)err[0];
+}
+__global__ void k_step_begin(unsigned long long *__restrict__ amax) { amax[1] = 0; }
 
 // Solves K x = b (extended vectors) with the factored band and FP64
 // iterative refinement against the block-sparse K; returns |b - K x| / |b|.
@@ -547,19 +550,21 @@ float elapsed(Ctx &c, int a, int b) {
 // the residual (it has reached the rounding floor of K x for this b, as
 // LAPACK's and UMFPACK's refinement stop).
 double solve_refined(Ctx &c, const double *d_b, double *d_x, int max_sweeps, double tol) {
-  const double bn = vec_norm2_masked(c, d_b);
+  vec_sumsq(c, c.nx, c.d_active, {{d_b, RED_B}});
   band_solve(c, d_b, d_x);
   double rel = 0.0, prev = 0.0;
   int sweeps = 0;
-  if (bn == 0.0) {
-    c.stats.last_relres = 0.0;
-    c.stats.refine_sweeps = 0;
-    return 0.0;
-  }
   for (;;) {
-    bsr_spmv(c, d_x, c.d_w);
-    vec_axpby(c, c.nx, 1.0, d_b, -1.0, c.d_w);  // w = b - K x
-    rel = vec_norm2_masked(c, c.d_w) / bn;
+    bsr_spmv(c, d_x, c.d_w, d_b);  // w = b - K x
+    vec_sumsq(c, c.nx, c.d_active, {{c.d_w, RED_W}, {d_x, RED_X}});
+    MAFEM_HIP(hipStreamSynchronize(c.stream));
+    const double bn = sqrt(c.h_red[RED_B]);
+    c.x_norm = sqrt(c.h_red[RED_X]);
+    if (bn == 0.0) {
+      rel = 0.0;
+      break;
+    }
+    rel = sqrt(c.h_red[RED_W]) / bn;
     if (rel < tol || sweeps >= max_sweeps || (sweeps > 0 && rel > 0.5 * prev)) break;
     prev = rel;
     band_solve(c, c.d_w, c.d_t);
@@ -631,6 +636,7 @@ void refactor(Ctx &c) {
 // (after any up-front factorization) bracket the factorization phase.
 double linear_solve(Ctx &c, const double *d_b, double *d_x) {
   const mafem_solver_opts &o = c.opts;
+  c.x_norm = -1.0;
   MAFEM_HIP(hipEventRecord(c.ev[2], c.stream));
   if (o.mode == MAFEM_SOLVER_DIRECT) {
     refactor(c);
@@ -651,6 +657,7 @@ double linear_solve(Ctx &c, const double *d_b, double *d_x) {
     ensure_krylov(c);
     int its = 0;
     const double rel2 = fgmres(c, d_b, d_x, &its);
+    c.x_norm = -1.0;
     c.stats.last_relres = rel2;
     return rel2;
   }
@@ -976,26 +983,33 @@ int mafem_time_step(mafem_ctx *ctx, double time, double dt, int32_t max_iter, in
     double eps = INFINITY;
     int it = 0;
     const int32_t nbs0 = c.n_band_solve, nf0 = c.n_factor, ng0 = c.n_gmres;
-    const int32_t np0 = read_pert(c);
+    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, c.stream, c.d_amax);
+    nd_begin_spans(c);
+    // an iteration's phase times, read once it is known to be over
+    auto phases = [&](const hipEvent_t *ev) {
+      st.assemble_us += 1e3 * elapsed(ev, 1, 2);
+      st.area_kernel_us += 1e3 * elapsed(ev, 8, 9);
+      st.factor_us += 1e3 * elapsed(ev, 2, 3);
+      st.solve_us += 1e3 * elapsed(ev, 3, 4);
+      st.update_us += 1e3 * elapsed(ev, 4, 5);
+    };
     int n_step = 0, n_sch = 0;
     double step_fl = 0.0, step_by = 0.0;
     c.step_timed = false;
-    MAFEM_HIP(hipEventRecord(c.ev[0], c.stream));
+    c.ev = c.evs;
+    MAFEM_HIP(hipEventRecord(c.evs[0], c.stream));
     while (it < max_iter) {
+      c.ev = c.evs + 12 * (it & 1);
       MAFEM_HIP(hipEventRecord(c.ev[1], c.stream));
       launch_assemble(c, time, dt);
       vec_scale(c, c.nt * TILE, -1.0, c.d_r, c.d_b);  // b = -r
-      linear_solve(c, c.d_b, c.d_x);
+      linear_solve(c, c.d_b, c.d_x);  // synchronizes
       MAFEM_HIP(hipEventRecord(c.ev[4], c.stream));
       apply_update(c, c.d_x, dt);
       MAFEM_HIP(hipEventRecord(c.ev[5], c.stream));
-      eps = vec_norm2_masked(c, c.d_x) / (double)c.nmdf;  // synchronizes
-      st.assemble_us += 1e3 * elapsed(c, 1, 2);
-      st.area_kernel_us += 1e3 * elapsed(c, 8, 9);
+      eps = (c.x_norm >= 0.0 ? c.x_norm : vec_norm2_masked(c, c.d_x)) / (double)c.nmdf;
+      if (it > 0) phases(c.evs + 12 * ((it - 1) & 1));
       st.n_assemble += 1;
-      st.factor_us += 1e3 * elapsed(c, 2, 3);
-      st.solve_us += 1e3 * elapsed(c, 3, 4);
-      st.update_us += 1e3 * elapsed(c, 4, 5);
       st.refine_sweeps += c.stats.refine_sweeps;
       if (c.step_timed) {  // on the context's stream: another thread may be capturing a graph
         unsigned long long sp[2];
@@ -1008,29 +1022,33 @@ int mafem_time_step(mafem_ctx *ctx, double time, double dt, int32_t max_iter, in
         }
         c.step_timed = false;
       }
-      if (c.ordering == 1) {
-        NdSpans sa, sb;
-        if (nd_read_spans(c, sa, sb)) {
-          st.step_kernel_us += sa.us;
-          n_step += sa.count;
-          step_fl += sa.flops;
-          step_by += sa.bytes;
-          st.schur_kernel_us += sb.us;
-          n_sch += sb.count;
-          st.schur_flops += sb.flops;
-          st.schur_bytes += sb.bytes;
-        }
-      }
       st.last_relres = c.stats.last_relres;
       if (eps_hist) eps_hist[it] = eps;
       ++it;
       if (!std::isfinite(eps)) break;
       if (eps < c.enr) break;
     }
-    MAFEM_HIP(hipEventRecord(c.ev[6], c.stream));
-    MAFEM_HIP(hipEventSynchronize(c.ev[6]));
-    check_sweeps(c);
+    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, c.stream, c.d_amax, c.d_sweep_err,
+                       c.h_red + RED_END);
+    nd_end_spans(c);
+    MAFEM_HIP(hipGetLastError());
+    MAFEM_HIP(hipEventRecord(c.evs[6], c.stream));
+    MAFEM_HIP(hipEventSynchronize(c.evs[6]));
+    if (it > 0) phases(c.ev);
+    c.ev = c.evs;
+    if (c.h_red[RED_END + 1] != 0.0) check_sweeps(c);
     st.total_us = 1e3 * elapsed(c, 0, 6);
+    NdSpans sa, sb;
+    if (nd_read_spans(c, sa, sb)) {
+      st.step_kernel_us += sa.us;
+      n_step += sa.count;
+      step_fl += sa.flops;
+      step_by += sa.bytes;
+      st.schur_kernel_us += sb.us;
+      n_sch += sb.count;
+      st.schur_flops += sb.flops;
+      st.schur_bytes += sb.bytes;
+    }
     st.newton_iters = it;
     st.n_band_solve = c.n_band_solve - nbs0;
     st.n_factor = c.n_factor - nf0;
@@ -1046,7 +1064,7 @@ int mafem_time_step(mafem_ctx *ctx, double time, double dt, int32_t max_iter, in
       st.schur_bytes /= n_sch;
     }
     st.sweep_groups = c.sweep_groups;
-    st.pivot_perturbations = read_pert(c) - np0;
+    st.pivot_perturbations = (int32_t)c.h_red[RED_END];
     fill_ordering_stats(c, st);
     c.stats = st;
     if (iters) *iters = it;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -23,6 +24,10 @@ constexpr int REC = 55;      // doubles per tabulated 2-D basis record
 constexpr int RECP = 56;     // padded record stride on the device
 constexpr int TILE = 64;     // band-LU tile edge
 constexpr int MAX_ADJ = 25;    // elements around the pulled one: (2 poly + 1)^2 for poly = 2
+// reduction scratch (d_red: partial sums of three vectors, then their tickets) and
+// results (h_red: pull force 0-5, end of a step 6-7, sums of squares, dot products)
+constexpr int NRED = 256;
+constexpr int RED_END = 6, RED_B = 8, RED_W = 9, RED_X = 10, RED_DOTS = 16, RED_N = RED_DOTS + 144;
 constexpr int SOLVE_RING = 72;  // solution tiles a sweep keeps in LDS (needs tb + 1 <= this)
 // Lanes per tangent column of the area-element kernel, by Motion (STATIC 1 ..
 // ALEVB 5; index 0 unused): each lane accumulates the rows of ceil(9 / parts)
@@ -56,7 +61,10 @@ struct Ctx {
   std::string err;
   int dev = 0;
   hipStream_t stream = nullptr;
-  hipEvent_t ev[12] = {};   // 0-6 phases, 8-9 area kernel
+  // 0-6 phases, 8-9 area kernel; two sets, so that an iteration's are read while
+  // the next one's are recorded
+  hipEvent_t evs[24] = {};
+  hipEvent_t *ev = evs;
 
   // sizes
   int64_t num1el = 0, num2el = 0, numel = 0, num1np = 0, num2np = 0, numnp = 0;
@@ -100,7 +108,8 @@ struct Ctx {
   double *d_r = nullptr, *d_x = nullptr, *d_w = nullptr, *d_t = nullptr, *d_b = nullptr;
   double *d_t2 = nullptr;        // band-solve intermediate
   double *d_red = nullptr;       // reduction scratch
-  double *h_red = nullptr;       // pinned host mirror of reduction results
+  double *h_red = nullptr;       // reduction results in pinned host memory
+  double x_norm = -1.0;          // |x| of the last solve over active entries (-1: not formed)
 
   // CSC export (1-based) over active DOFs, built on first use (nnz < 0 before)
   std::vector<int64_t> h_ID, h_eq;
@@ -343,22 +352,32 @@ int nd_prec(const Ctx &c);       // storage precision of the fronts (0: none)
 int nd_fronts(const Ctx &c);     // fronts of the elimination tree (0: not built)
 int nd_steps(const Ctx &c);      // dependent tile steps of one factorization
 double nd_flops(const Ctx &c);   // algorithmic FLOPs of one factorization
-// durations (sum, us) / count / FLOPs / bytes of the last factorization's step launches
+// durations (sum, us) / count / FLOPs / bytes of a kind of launch
 struct NdSpans {
   double us = 0, flops = 0, bytes = 0;  // sums over the timed launches
   int count = 0;
 };
+// the factorizations from nd_begin_spans on: nd_end_spans has their durations put
+// into host memory, nd_read_spans reads them once the stream has been waited for
+void nd_begin_spans(Ctx &c);
+void nd_end_spans(Ctx &c);
 bool nd_read_spans(Ctx &c, NdSpans &step, NdSpans &schur);
 int64_t nd_bytes(const Ctx &c);  // bytes of factor storage
-void bsr_spmv(Ctx &c, const double *d_x, double *d_y);
+void bsr_spmv(Ctx &c, const double *d_x, double *d_y, const double *d_b = nullptr);
 void vec_axpby(Ctx &c, int64_t n, double a, const double *x, double b, double *y);
 void vec_zero(Ctx &c, int64_t n, double *y);
 void vec_scale(Ctx &c, int64_t n, double a, const double *x, double *y);
 double vec_norm2_masked(Ctx &c, const double *x);   // active entries only, blocking
-double vec_norm2(Ctx &c, const double *x, int64_t n);  // all entries, blocking
+// sums of squares of up to three vectors (of the entries where mask is set) into
+// c.h_red[slot], valid once the stream has been waited for
+struct SumSqOf {
+  const double *x;
+  int slot;
+};
+void vec_sumsq(Ctx &c, int64_t n, const uint8_t *mask, std::initializer_list<SumSqOf> v);
 // multi-vector kernels of the Krylov solver (vec.hip)
-void vec_mdot(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *w, double *h_out);
-void vec_mcomb(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *h_coef, double alpha, double *w);
+void vec_mdot(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *w, double *d_out, double *h_out);
+void vec_mcomb(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *d_coef, double alpha, double *w);
 // Krylov solver (krylov.hip): K x = b, x overwritten; returns |b - K x| / |b|
 double fgmres(Ctx &c, const double *d_b, double *d_x, int *iters);
 void ensure_krylov(Ctx &c);

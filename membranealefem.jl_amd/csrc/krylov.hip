@@ -29,7 +29,7 @@ void ensure_krylov(Ctx &c) {
   MAFEM_HIP(hipMemset(c.d_V, 0, sizeof(double) * ld * (m + 1)));
   MAFEM_HIP(hipMemset(c.d_Z, 0, sizeof(double) * ld * m));
   if (!c.d_h) {
-    MAFEM_HIP(hipMalloc((void **)&c.d_h, sizeof(double) * 72));
+    MAFEM_HIP(hipMalloc((void **)&c.d_h, sizeof(double) * 144));
     MAFEM_HIP(hipMalloc((void **)&c.d_coef, sizeof(double) * 72));
     MAFEM_HIP(hipMalloc((void **)&c.d_mdot_part, sizeof(double) * 72 * 256));
   }
@@ -44,20 +44,21 @@ double fgmres(Ctx &c, const double *d_b, double *d_x, int *iters_out) {
   const int maxit = std::max(1, (int)c.opts.max_iters);
   double *V = c.d_V, *Z = c.d_Z, *w = c.d_w;
   int total = 0;
-  const double bn = vec_norm2(c, d_b, n);
-  if (bn == 0.0) {
-    vec_zero(c, ld, d_x);
-    *iters_out = 0;
-    return 0.0;
-  }
+  vec_sumsq(c, n, nullptr, {{d_b, RED_B}});
   band_solve(c, d_b, d_x);  // x0 = M^-1 b
-  std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m), sn(m), g(m + 1), h(m + 1), h2(m + 1),
-      y(m);
+  const double *dots = c.h_red + RED_DOTS;  // 2 x 72 dot products, pinned
+  std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m), sn(m), g(m + 1), h(m + 1), y(m);
   double rel = 0.0;
   for (;;) {
-    bsr_spmv(c, d_x, w);
-    vec_axpby(c, n, 1.0, d_b, -1.0, w);  // w = b - K x
-    const double beta = vec_norm2(c, w, n);
+    bsr_spmv(c, d_x, w, d_b);  // w = b - K x
+    vec_sumsq(c, n, nullptr, {{w, RED_W}});
+    MAFEM_HIP(hipStreamSynchronize(c.stream));
+    const double bn = sqrt(c.h_red[RED_B]), beta = sqrt(c.h_red[RED_W]);
+    if (bn == 0.0) {
+      vec_zero(c, ld, d_x);
+      *iters_out = 0;
+      return 0.0;
+    }
     rel = beta / bn;
     if (!(rel > rtol) || total >= maxit) break;
     vec_scale(c, n, 1.0 / beta, w, V);
@@ -68,12 +69,16 @@ double fgmres(Ctx &c, const double *d_b, double *d_x, int *iters_out) {
       band_solve(c, V + j * ld, Z + j * ld);
       double *vn = V + (j + 1) * ld;
       bsr_spmv(c, Z + j * ld, vn);
-      vec_mdot(c, n, j + 1, V, ld, vn, h.data());
-      vec_mcomb(c, n, j + 1, V, ld, h.data(), -1.0, vn);
-      vec_mdot(c, n, j + 1, V, ld, vn, h2.data());
-      vec_mcomb(c, n, j + 1, V, ld, h2.data(), -1.0, vn);
-      for (int k = 0; k <= j; ++k) h[k] += h2[k];
-      const double hn = vec_norm2(c, vn, n);
+      // classical Gram-Schmidt, twice, its coefficients kept on the device
+      for (int pass = 0; pass < 2; ++pass) {
+        double *coef = c.d_h + 72 * pass;
+        vec_mdot(c, n, j + 1, V, ld, vn, coef, c.h_red + RED_DOTS + 72 * pass);
+        vec_mcomb(c, n, j + 1, V, ld, coef, -1.0, vn);
+      }
+      vec_sumsq(c, n, nullptr, {{vn, RED_W}});
+      MAFEM_HIP(hipStreamSynchronize(c.stream));
+      for (int k = 0; k <= j; ++k) h[k] = dots[k] + dots[72 + k];
+      const double hn = sqrt(c.h_red[RED_W]);
       if (hn > 0.0) vec_scale(c, n, 1.0 / hn, vn, vn);
       for (int k = 0; k < j; ++k) {
         const double a = h[k], b2 = h[k + 1];
@@ -98,7 +103,11 @@ double fgmres(Ctx &c, const double *d_b, double *d_x, int *iters_out) {
       for (int l = k + 1; l < j; ++l) s -= H[(size_t)k * m + l] * y[l];
       y[k] = s / H[(size_t)k * m + k];
     }
-    if (j > 0) vec_mcomb(c, n, j, Z, ld, y.data(), 1.0, d_x);
+    if (j > 0) {
+      MAFEM_HIP(hipMemcpyAsync(c.d_coef, y.data(), sizeof(double) * j, hipMemcpyHostToDevice,
+                               c.stream));
+      vec_mcomb(c, n, j, Z, ld, c.d_coef, 1.0, d_x);
+    }
   }
   c.n_gmres += total;
   *iters_out = total;

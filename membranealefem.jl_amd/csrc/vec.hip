@@ -9,13 +9,15 @@
 namespace mafem {
 
 
-// y = K x over the node blocks (ndf <= 8): eight lanes per row, lane c takes
-// column c of every block of the row's node (a wavefront reads whole blocks
-// coalesced), then the eight partial sums are added in a fixed tree
+// y = K x over the node blocks (ndf <= 8), or y = b - K x where b is given: eight
+// lanes per row, lane c takes column c of every block of the row's node (a
+// wavefront reads whole blocks coalesced), then the eight partial sums are added
+// in a fixed tree
 __global__ __launch_bounds__(256) void k_spmv(int64_t nx, int ndf, const int32_t *__restrict__ rowptr,
                                               const int32_t *__restrict__ colidx,
                                               const double *__restrict__ bsr,
                                               const double *__restrict__ x,
+                                              const double *__restrict__ b,
                                               double *__restrict__ y) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t R = t >> 3;
@@ -31,7 +33,7 @@ __global__ __launch_bounds__(256) void k_spmv(int64_t nx, int ndf, const int32_t
   s += __shfl_xor(s, 1, 8);
   s += __shfl_xor(s, 2, 8);
   s += __shfl_xor(s, 4, 8);
-  if (c == 0) y[R] = s;
+  if (c == 0) y[R] = b ? b[R] - s : s;
 }
 
 __global__ __launch_bounds__(256) void k_axpby(int64_t n, double a, const double *__restrict__ x,
@@ -40,41 +42,58 @@ __global__ __launch_bounds__(256) void k_axpby(int64_t n, double a, const double
   if (t < n) y[t] = a * x[t] + b * y[t];
 }
 
-constexpr int NRED = 256;  // fixed partition: deterministic reduction order
-
 __global__ __launch_bounds__(256) void k_zero(int64_t n, double *__restrict__ x) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t < n) x[t] = 0.0;
 }
 
-__global__ __launch_bounds__(256) void k_sumsq_partial(int64_t n, const double *__restrict__ x,
-                                                       const uint8_t *__restrict__ mask,
-                                                       double *__restrict__ part) {
+__device__ __forceinline__ double tree_sum(double v) {
   __shared__ double s[256];
-  double acc = 0.0;
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)NRED * 256) {
-    const double v = (mask == nullptr || mask[t]) ? x[t] : 0.0;
-    acc = fma(v, v, acc);
-  }
-  s[threadIdx.x] = acc;
+  s[threadIdx.x] = v;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+  return s[0];
 }
 
-__global__ __launch_bounds__(256) void k_sum_final(const double *__restrict__ part,
-                                                   double *__restrict__ out) {
-  __shared__ double s[256];
-  s[threadIdx.x] = part[threadIdx.x];
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
+// Sums of squares of up to three vectors (blockIdx.y), each over at most NRED
+// blocks; the last block of a vector to arrive adds the partials in their order
+// and writes the sum to out[slot], pinned host memory (a launch for the final sum
+// and a copy of eight bytes took 4 us each).
+struct SumSq {
+  const double *x[3];
+  int32_t slot[3];
+};
+__global__ __launch_bounds__(256) void k_sumsq(int64_t n, SumSq v, const uint8_t *__restrict__ mask,
+                                               double *__restrict__ part,
+                                               unsigned *__restrict__ ticket,
+                                               double *__restrict__ out) {
+  __shared__ unsigned mine;
+  const int k = (int)blockIdx.y;
+  const double *__restrict__ x = v.x[k];
+  part += k * NRED;
+  double acc = 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+    const double e = (mask == nullptr || mask[t]) ? x[t] : 0.0;
+    acc = fma(e, e, acc);
   }
-  if (threadIdx.x == 0) out[0] = s[0];
+  const double s = tree_sum(acc);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(&part[blockIdx.x], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mine = __hip_atomic_fetch_add(&ticket[k], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (mine + 1 != gridDim.x) return;
+  const double p = threadIdx.x < gridDim.x
+                       ? __hip_atomic_load(&part[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                       : 0.0;
+  const double r = tree_sum(p);
+  if (threadIdx.x == 0) {
+    out[v.slot[k]] = r;
+    ticket[k] = 0;
+  }
 }
 
 // cps += Δcps; xms += Δt Δcps[:, motion]  (FiniteElement.jl:41-46)
@@ -102,9 +121,10 @@ __global__ __launch_bounds__(256) void k_update_state(int64_t numnp, int ndf, in
 
 static inline unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-void bsr_spmv(Ctx &c, const double *d_x, double *d_y) {
+// y = K x, or b - K x where b is given
+void bsr_spmv(Ctx &c, const double *d_x, double *d_y, const double *d_b) {
   hipLaunchKernelGGL(k_spmv, dim3(nblk(8 * c.nx)), dim3(256), 0, c.stream, c.nx, c.ndf, c.d_rowptr,
-                     c.d_colidx, c.d_bsr, d_x, d_y);
+                     c.d_colidx, c.d_bsr, d_x, d_b, d_y);
   MAFEM_HIP(hipGetLastError());
 }
 
@@ -129,15 +149,23 @@ void vec_axpby(Ctx &c, int64_t n, double a, const double *x, double b, double *y
   MAFEM_HIP(hipGetLastError());
 }
 
-double vec_norm2_masked(Ctx &c, const double *x) {
-  hipLaunchKernelGGL(k_sumsq_partial, dim3(NRED), dim3(256), 0, c.stream, c.nx, x, c.d_active,
-                     c.d_red);
-  hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, c.stream, c.d_red, c.d_red + NRED);
+void vec_sumsq(Ctx &c, int64_t n, const uint8_t *mask, std::initializer_list<SumSqOf> v) {
+  SumSq a{};
+  int k = 0;
+  for (const SumSqOf &e : v) {
+    a.x[k] = e.x;
+    a.slot[k++] = e.slot;
+  }
+  const unsigned nb = std::min<unsigned>(NRED, std::max(1u, nblk(n)));
+  hipLaunchKernelGGL(k_sumsq, dim3(nb, k), dim3(256), 0, c.stream, n, a, mask, c.d_red,
+                     (unsigned *)(c.d_red + 3 * NRED), c.h_red);
   MAFEM_HIP(hipGetLastError());
-  MAFEM_HIP(hipMemcpyAsync(c.h_red, c.d_red + NRED, sizeof(double), hipMemcpyDeviceToHost,
-                           c.stream));
+}
+
+double vec_norm2_masked(Ctx &c, const double *x) {
+  vec_sumsq(c, c.nx, c.d_active, {{x, RED_X}});
   MAFEM_HIP(hipStreamSynchronize(c.stream));
-  return sqrt(c.h_red[0]);
+  return sqrt(c.h_red[RED_X]);
 }
 
 void apply_update(Ctx &c, const double *d_du, double dt) {
@@ -169,7 +197,8 @@ __global__ __launch_bounds__(256) void k_mdot_partial(int64_t n, const double *_
 }
 
 __global__ __launch_bounds__(256) void k_mdot_final(const double *__restrict__ part,
-                                                    double *__restrict__ out) {
+                                                    double *__restrict__ out,
+                                                    double *__restrict__ host) {
   __shared__ double s[256];
   const int k = blockIdx.x;
   s[threadIdx.x] = part[(int64_t)k * NRED + threadIdx.x];
@@ -178,7 +207,7 @@ __global__ __launch_bounds__(256) void k_mdot_final(const double *__restrict__ p
     if (threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[k] = s[0];
+  if (threadIdx.x == 0) out[k] = host[k] = s[0];
 }
 
 // w += alpha * sum_k coef[k] V_k
@@ -192,35 +221,20 @@ __global__ __launch_bounds__(256) void k_mcomb(int64_t n, int nvec, const double
   w[t] = fma(alpha, s, w[t]);
 }
 
-double vec_norm2(Ctx &c, const double *x, int64_t n) {
-  hipLaunchKernelGGL(k_sumsq_partial, dim3(NRED), dim3(256), 0, c.stream, n, x,
-                     (const uint8_t *)nullptr, c.d_red);
-  hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, c.stream, c.d_red, c.d_red + NRED);
-  MAFEM_HIP(hipGetLastError());
-  MAFEM_HIP(hipMemcpyAsync(c.h_red, c.d_red + NRED, sizeof(double), hipMemcpyDeviceToHost,
-                           c.stream));
-  MAFEM_HIP(hipStreamSynchronize(c.stream));
-  return sqrt(c.h_red[0]);
-}
-
-// h_out (host) = V^T w for the first nvec columns; blocking
+// out = V^T w for the first nvec columns, on the device and in pinned host memory
 void vec_mdot(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *w,
-              double *h_out) {
+              double *d_out, double *h_out) {
   hipLaunchKernelGGL(k_mdot_partial, dim3(NRED, nvec), dim3(256), 0, c.stream, n, V, ld, w,
                      c.d_mdot_part);
-  hipLaunchKernelGGL(k_mdot_final, dim3(nvec), dim3(256), 0, c.stream, c.d_mdot_part, c.d_h);
+  hipLaunchKernelGGL(k_mdot_final, dim3(nvec), dim3(256), 0, c.stream, c.d_mdot_part, d_out, h_out);
   MAFEM_HIP(hipGetLastError());
-  MAFEM_HIP(hipMemcpyAsync(h_out, c.d_h, sizeof(double) * nvec, hipMemcpyDeviceToHost, c.stream));
-  MAFEM_HIP(hipStreamSynchronize(c.stream));
 }
 
-// w += alpha * V coef, coef given on the host
-void vec_mcomb(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *h_coef,
+// w += alpha * V coef
+void vec_mcomb(Ctx &c, int64_t n, int nvec, const double *V, int64_t ld, const double *d_coef,
                double alpha, double *w) {
-  MAFEM_HIP(hipMemcpyAsync(c.d_coef, h_coef, sizeof(double) * nvec, hipMemcpyHostToDevice,
-                           c.stream));
-  hipLaunchKernelGGL(k_mcomb, dim3(nblk(n)), dim3(256), 0, c.stream, n, nvec, V, ld, c.d_coef,
-                     alpha, w);
+  hipLaunchKernelGGL(k_mcomb, dim3(nblk(n)), dim3(256), 0, c.stream, n, nvec, V, ld, d_coef, alpha,
+                     w);
   MAFEM_HIP(hipGetLastError());
 }
 
