@@ -48,7 +48,7 @@ void free_all(Ctx &c) {
                   c.d_dbt,  c.d_bufns,  c.d_edges,   c.d_kel,     c.d_rel,    c.d_rowptr,
                   c.d_colidx, c.d_brow, c.d_bsr,     c.d_gptr,    c.d_gsrc,   c.d_rptr,
                   c.d_rsrc, c.d_r,      c.d_x,       c.d_w,       c.d_t,      c.d_b,
-                  c.d_red,  c.d_csc_src, c.d_csc_val, c.d_eq,     c.d_band,   c.d_linv,
+                  c.d_red,  c.d_csc_src, c.d_eq,     c.d_band,   c.d_linv,
                   c.d_uinv, c.d_piv,  c.d_V,       c.d_Z,       c.d_h,      c.d_coef,
                   c.d_mdot_part, c.d_t2, c.d_presc_idx, c.d_presc_val, c.d_s1, c.d_s2,
                   c.d_sweep_err, c.d_pf_el, c.d_pf_slot, c.d_pf_rel,
@@ -58,6 +58,7 @@ void free_all(Ctx &c) {
     if (p) (void)hipFree(p);
   nd_free(c);
   if (c.h_red) (void)hipHostFree(c.h_red);
+  if (c.h_stage) (void)hipHostFree(c.h_stage);
   for (auto &e : c.evs)
     if (e) (void)hipEventDestroy(e);
   if (c.stream) (void)hipStreamDestroy(c.stream);
@@ -510,7 +511,6 @@ void ensure_csc(Ctx &c) {
   c.h_colptr[nmdf] = (int64_t)c.h_rowval.size() + 1;
   const int64_t nnz = (int64_t)c.h_rowval.size();
   c.d_csc_src = dupload(c, csc_src);
-  c.d_csc_val = dalloc<double>(c, nnz);
   c.nnz = nnz;
 }
 
@@ -527,6 +527,49 @@ __global__ void k_scatter_idx(int64_t n, const int64_t *__restrict__ idx,
 }
 
 inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+// dst (host memory of the caller) = src[idx[0 .. n - 1]]
+struct Export {
+  int64_t n;
+  const int64_t *idx;
+  const double *src;
+  double *dst;
+};
+
+// The values go to the host in chunks through pinned memory that the gather writes
+// itself: the next chunk crosses the bus while the host copies this one (copies
+// into pageable memory ran at 16 GB/s: 31x24 EUL 440 us for its 7.2 MB).
+void export_values(Ctx &c, const std::vector<Export> &out) {
+  struct Chunk {
+    double *dst;
+    int64_t n;
+  };
+  if (!c.h_stage) {
+    std::lock_guard<std::mutex> no_capture(capture_mutex());
+    MAFEM_HIP(hipHostMalloc((void **)&c.h_stage, sizeof(double) * 2 * EXPORT_CHUNK,
+                            hipHostMallocDefault));
+  }
+  Chunk fly[2] = {};
+  int k = 0;
+  auto land = [&](int i) {
+    if (fly[i].n == 0) return;
+    MAFEM_HIP(hipEventSynchronize(c.ev[10 + i]));
+    std::memcpy(fly[i].dst, c.h_stage + i * EXPORT_CHUNK, sizeof(double) * fly[i].n);
+    fly[i].n = 0;
+  };
+  for (const Export &e : out)
+    for (int64_t o = 0; o < e.n; o += EXPORT_CHUNK, k ^= 1) {
+      const int64_t n = std::min(EXPORT_CHUNK, e.n - o);
+      land(k);
+      hipLaunchKernelGGL(k_gather_idx, dim3(nb256(n)), dim3(256), 0, c.stream, n, e.idx + o, e.src,
+                         c.h_stage + k * EXPORT_CHUNK);
+      MAFEM_HIP(hipGetLastError());
+      MAFEM_HIP(hipEventRecord(c.ev[10 + k], c.stream));
+      fly[k] = {e.dst + o, n};
+    }
+  land(k);
+  land(k ^ 1);
+}
 
 float elapsed(const hipEvent_t *ev, int a, int b) {
   float ms = 0.f;
@@ -885,9 +928,7 @@ int mafem_set_dof_ids(mafem_ctx *ctx, const int64_t *ID, int64_t nmdf) {
     c.h_eq = eq;
     // the CSC export pattern follows the numbering: rebuilt on next use
     if (c.d_csc_src) (void)hipFree(c.d_csc_src);
-    if (c.d_csc_val) (void)hipFree(c.d_csc_val);
     c.d_csc_src = nullptr;
-    c.d_csc_val = nullptr;
     c.nnz = -1;
     c.h_colptr.clear();
     c.h_rowval.clear();
@@ -922,18 +963,10 @@ int mafem_assemble(mafem_ctx *ctx, double time, double dt, double *r, int64_t *c
     MAFEM_HIP(hipEventRecord(c.ev[0], c.stream));
     launch_assemble(c, time, dt);
     MAFEM_HIP(hipEventRecord(c.ev[1], c.stream));
-    if (r) {
-      hipLaunchKernelGGL(k_gather_idx, dim3(nb256(c.nmdf)), dim3(256), 0, c.stream, c.nmdf, c.d_eq,
-                         c.d_r, c.d_w);
-      MAFEM_HIP(hipGetLastError());
-      MAFEM_HIP(hipMemcpyAsync(r, c.d_w, sizeof(double) * c.nmdf, hipMemcpyDeviceToHost, c.stream));
-    }
-    if (nzval) {
-      hipLaunchKernelGGL(k_gather_idx, dim3(nb256(c.nnz)), dim3(256), 0, c.stream, c.nnz,
-                         c.d_csc_src, c.d_bsr, c.d_csc_val);
-      MAFEM_HIP(hipGetLastError());
-      MAFEM_HIP(hipMemcpyAsync(nzval, c.d_csc_val, sizeof(double) * c.nnz, hipMemcpyDeviceToHost, c.stream));
-    }
+    std::vector<Export> out;
+    if (r) out.push_back({c.nmdf, c.d_eq, c.d_r, r});
+    if (nzval) out.push_back({c.nnz, c.d_csc_src, c.d_bsr, nzval});
+    export_values(c, out);
     MAFEM_HIP(hipStreamSynchronize(c.stream));
     if (colptr) std::memcpy(colptr, c.h_colptr.data(), sizeof(int64_t) * (c.nmdf + 1));
     if (rowval) std::memcpy(rowval, c.h_rowval.data(), sizeof(int64_t) * c.nnz);

@@ -26,6 +26,7 @@ constexpr int TILE = 64;     // band-LU tile edge
 constexpr int MAX_ADJ = 25;    // elements around the pulled one: (2 poly + 1)^2 for poly = 2
 // reduction scratch (d_red: partial sums of three vectors, then their tickets) and
 // results (h_red: pull force 0-5, end of a step 6-7, sums of squares, dot products)
+constexpr int64_t EXPORT_CHUNK = 1 << 18;
 constexpr int NRED = 256;
 constexpr int RED_END = 6, RED_B = 8, RED_W = 9, RED_X = 10, RED_DOTS = 16, RED_N = RED_DOTS + 144;
 constexpr int SOLVE_RING = 72;  // solution tiles a sweep keeps in LDS (needs tb + 1 <= this)
@@ -117,7 +118,7 @@ struct Ctx {
   int64_t nnz = -1;
   std::vector<int64_t> h_colptr, h_rowval;
   int64_t *d_csc_src = nullptr;  // BSR value index of each CSC entry
-  double *d_csc_val = nullptr;
+  double *h_stage = nullptr;     // two pinned chunks of EXPORT_CHUNK values (exports)
   int64_t *d_eq = nullptr;       // extended index of each equation (nmdf)
 
   // band LU (storage precision band_prec: 64 or 32; allocated on first use)

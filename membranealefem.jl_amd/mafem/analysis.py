@@ -73,7 +73,7 @@ class DeviceMesh:
             raise L.LibError(rc, self.lib.mafem_last_error(None).decode())
         self.h = h
         self.nmdf = m.nmdf
-        self._nnz = None
+        self._nnz = self._pattern = None
 
     # -- plumbing
     def _check(self, rc):
@@ -122,7 +122,7 @@ class DeviceMesh:
         nmdf = int(a.max())
         self._check(self.lib.mafem_set_dof_ids(self.h, L.ptr(a, L.i64p), nmdf))
         self.nmdf = nmdf
-        self._nnz = None
+        self._nnz = self._pattern = None
 
     # -- hot path
     def nnz(self):
@@ -139,12 +139,20 @@ class DeviceMesh:
             self._check(self.lib.mafem_assemble(self.h, time, dt, L.ptr(r, L.f64p), None, None,
                                                 None))
             return r, None
+        v = np.empty(nz)
+        if self._pattern is not None:
+            self._check(self.lib.mafem_assemble(self.h, time, dt, L.ptr(r, L.f64p), None, None,
+                                                L.ptr(v, L.f64p)))
+            rows, cols = self._pattern
+            return r, sps.csc_matrix((v, rows.copy(), cols.copy()), shape=(n, n))
         cp = np.zeros(n + 1, dtype=np.int64)
         rv = np.zeros(nz, dtype=np.int64)
-        v = np.zeros(nz)
         self._check(self.lib.mafem_assemble(self.h, time, dt, L.ptr(r, L.f64p), L.ptr(cp, L.i64p),
                                             L.ptr(rv, L.i64p), L.ptr(v, L.f64p)))
         K = sps.csc_matrix((v, rv - 1, cp - 1), shape=(n, n))
+        # the pattern belongs to the mesh and the equation numbering: later
+        # matrices take it as scipy keeps it
+        self._pattern = K.indices.copy(), K.indptr.copy()
         return r, K
 
     def solve(self, rhs):
