@@ -392,6 +392,8 @@ void build(Ctx &c, const mafem_mesh_desc *m, const mafem_params *p) {
     else if (std::strcmp(e, "nd") == 0) c.ordering = 1;
   }
 
+  MAFEM_HIP(hipDeviceGetAttribute(&c.cus, hipDeviceAttributeMultiprocessorCount, c.dev));
+
   // device allocations and uploads
   MAFEM_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   for (auto &e : c.evs) MAFEM_HIP(hipEventCreate(&e));

@@ -935,13 +935,15 @@ __global__ __launch_bounds__(256) void kb_predict(Seg sg, const PatchDev *__rest
   predict_at((blockIdx.x - sg.blk0[p]) * 256 + threadIdx.x, d.numnp, d.mm, d.cps, dts[p], d.xms);
 }
 
-static hipError_t launch_area(Ctx &c, double dt) {
-  const int64_t lanes = c.numel * c.ne * area_parts(c.motion);
-  const dim3 grid((unsigned)((lanes + 255) / 256));
-#define AREA(MO)                                                                        \
-  hipLaunchKernelGGL(k_area<MO>, grid, dim3(256), 0, c.stream, c.numel, c.numnp, c.d_ix, \
-                     c.d_uel, c.d_active, c.d_xms, c.d_cps, c.d_ufns, c.d_dbt, c.phys, dt, \
-                     c.d_kel, c.d_rel)
+// elements e0 .. e0 + n - 1
+template <int P>
+static hipError_t launch_area_p(Ctx &c, double dt, int64_t e0, int64_t n) {
+  const dim3 grid((unsigned)((n * c.ne * P + 255) / 256));
+  const int64_t ne = c.ne;
+#define AREA(MO)                                                                               \
+  hipLaunchKernelGGL((k_area<MO, P>), grid, dim3(256), 0, c.stream, n, c.numnp, c.d_ix + 9 * e0, \
+                     c.d_uel + e0, c.d_active, c.d_xms, c.d_cps, c.d_ufns, c.d_dbt, c.phys, dt,  \
+                     c.d_kel + e0 * ne * ne, c.d_rel + e0 * ne)
   switch (c.motion) {
     case STATIC: AREA(STATIC); break;
     case LAG: AREA(LAG); break;
@@ -952,6 +954,27 @@ static hipError_t launch_area(Ctx &c, double dt) {
   }
 #undef AREA
   return hipGetLastError();
+}
+
+// One block is resident per CU (its 260 to 430 registers), so with one lane per
+// column the kernel takes whole rounds of 62 us (ALEVB; LAG 43) however few
+// blocks the last one has.  The elements beyond the full rounds go to a launch of
+// their own with as many lanes per column, 9, 3 or 2, as still make one round: it
+// takes 25, 33 or 45 us (LAG 21, 27, 35).  ALEVB 8x8 57 -> 26 us, 17x13 60 -> 36, 20x20
+// 68 -> 50, 32x32 124 -> 100; LAG 8x8 41 -> 21, 96x80 216 -> 202.
+static hipError_t launch_area(Ctx &c, double dt) {
+  const int64_t cus = c.cus, lanes = c.numel * c.ne;
+  const int64_t rounds = (lanes + 255) / 256 / cus;
+  const int64_t e0 = std::min(c.numel, rounds * cus * 256 / c.ne), n = c.numel - e0;
+  const int64_t b = (n * c.ne + 255) / 256;
+  if (2 * b > cus) return launch_area_p<1>(c, dt, 0, c.numel);
+  if (e0 > 0) {
+    const hipError_t e = launch_area_p<1>(c, dt, 0, e0);
+    if (e != hipSuccess || n == 0) return e;
+  }
+  if ((n * c.ne * 9 + 255) / 256 <= cus) return launch_area_p<9>(c, dt, e0, n);
+  if ((n * c.ne * 3 + 255) / 256 <= cus) return launch_area_p<3>(c, dt, e0, n);
+  return launch_area_p<2>(c, dt, e0, n);
 }
 
 static hipError_t launch_edge(Ctx &c, double time, double dt) {

@@ -34,7 +34,8 @@ constexpr int SOLVE_RING = 72;  // solution tiles a sweep keeps in LDS (needs tb
 // ALEVB 5; index 0 unused): each lane accumulates the rows of ceil(9 / parts)
 // nodes.  With the Gauss points' values shared through LDS one lane per column
 // fits the registers without spills and is the fastest split for every motion
-// at 64x64 (ALEVB 338 us against 463 us with 3 and 918 us with 9).
+// where the chip is filled several times over (64x64 ALEVB 338 us against 463 us
+// with 3 and 918 us with 9); launch_area splits what does not fill it.
 constexpr int AREA_PARTS[6] = {1, 1, 1, 1, 1, 1};
 inline int area_parts(int motion) { return motion >= 1 && motion <= 5 ? AREA_PARTS[motion] : 1; }
 
@@ -66,6 +67,7 @@ struct Ctx {
   // the next one's are recorded
   hipEvent_t evs[24] = {};
   hipEvent_t *ev = evs;
+  int cus = 256;                // compute units of the device
 
   // sizes
   int64_t num1el = 0, num2el = 0, numel = 0, num1np = 0, num2np = 0, numnp = 0;
@@ -299,7 +301,7 @@ struct BatchPlan {
   BatchFlags f{};
   std::vector<int> motions;         // motions present
   std::vector<Seg> area, edge;      // per motion present
-  Seg bsr, vec, node;
+  Seg bsr, vec, row, node;
 };
 
 // batched launch sequences (assemble.hip, band.hip, vec.hip)
