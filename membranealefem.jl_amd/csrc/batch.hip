@@ -186,17 +186,19 @@ void build_plan(mafem_batch &b) {
     B.area.push_back(make_seg(b, ba, 256));
     B.edge.push_back(make_seg(b, be, 256));
   }
-  std::vector<int64_t> bb(P), bv(P), bn(P);
+  std::vector<int64_t> bb(P), bv(P), br(P), bn(P);
   for (int p = 0; p < P; ++p) {
     const PatchDev &d = b.h_pd[p];
     bb[p] = cdiv(d.nnzb * d.ndf * d.ndf, 256);
     bv[p] = cdiv(d.nt * TILE, 256);
+    br[p] = d.nt * TILE / 32;
     bn[p] = cdiv(d.numnp, 256);
   }
   B.bsr = make_seg(b, bb, 256);
   B.vec = make_seg(b, bv, 256);
+  B.row = make_seg(b, br, 256);
   B.node = make_seg(b, bn, 256);
-  B.f.part = balloc<double>(b, std::max<int64_t>(B.vec.nblk, 1));
+  B.f.part = balloc<double>(b, std::max<int64_t>(B.row.nblk, 1));
   B.f.part2 = balloc<double>(b, std::max<int64_t>((int64_t)B.vec.nblk * (B.m + 1), 1));
 }
 

@@ -312,29 +312,40 @@ __global__ __launch_bounds__(256) void kb_solve_begin_fin(Seg sg, const PatchDev
   }
 }
 
+// (K x)_R of a patch, 32 rows a block (segment B.row), eight lanes per row as in
+// k_spmv (a lane per row reads 8-byte pieces 64 apart: 54 us a product of 16 patches
+// of 16 to 40 a side, 71 a residual); in all eight lanes
+__device__ __forceinline__ double row_spmv(const PatchDev &d, const double *__restrict__ x,
+                                           int64_t R) {
+  const int c = (int)(threadIdx.x & 7), bb = d.ndf * d.ndf;
+  double s = 0.0;
+  if (R < d.nx && c < d.ndf) {
+    const int64_t p = R / d.ndf;
+    const double *row = d.bsr + (R % d.ndf) * d.ndf + c;
+    for (int32_t k = d.rowptr[p]; k < d.rowptr[p + 1]; ++k)
+      s = fma(row[(int64_t)k * bb], x[(int64_t)d.colidx[k] * d.ndf + c], s);
+  }
+  s += __shfl_xor(s, 1, 8);
+  s += __shfl_xor(s, 2, 8);
+  s += __shfl_xor(s, 4, 8);
+  return s;
+}
+__device__ __forceinline__ int64_t row_blocks(const PatchDev &d) { return d.nt * TILE / 32; }
+
 // w = b - K x in FP64 against the block-sparse tangent; partial |w|^2
 __global__ __launch_bounds__(256) void kb_resid(Seg sg, const PatchDev *__restrict__ pd,
                                                 const uint8_t *__restrict__ mask,
                                                 double *__restrict__ part) {
-  const VecAt at = vec_at(sg);
+  const int p = sg.map[blockIdx.x];
   double a = 0.0;
-  if (mask[at.p]) {
-    const PatchDev &d = pd[at.p];
-    const int64_t R = at.t;
-    if (R < d.nx) {
-      const int64_t q = R / d.ndf;
-      const int r = (int)(R % d.ndf), bb = d.ndf * d.ndf;
-      double s = 0.0;
-      for (int32_t k = d.rowptr[q]; k < d.rowptr[q + 1]; ++k) {
-        const double *blk = d.bsr + (int64_t)k * bb + r * d.ndf;
-        const double *xv = d.x + (int64_t)d.colidx[k] * d.ndf;
-        for (int c = 0; c < d.ndf; ++c) s = fma(blk[c], xv[c], s);
-      }
-      const double wv = d.b[R] - s;
+  if (mask[p]) {
+    const PatchDev &d = pd[p];
+    const int64_t R = (int64_t)(blockIdx.x - sg.blk0[p]) * 32 + (threadIdx.x >> 3);
+    const double s = row_spmv(d, d.x, R);
+    if ((threadIdx.x & 7) == 0) {
+      const double wv = R < d.nx ? d.b[R] - s : 0.0;
       d.w[R] = wv;
-      if (d.active[R]) a = wv * wv;
-    } else if (R < d.nt * TILE) {
-      d.w[R] = 0.0;
+      if (R < d.nx && d.active[R]) a = wv * wv;
     }
   }
   a = block_sum(a);
@@ -347,7 +358,7 @@ __global__ __launch_bounds__(256) void kb_cycle_start(Seg sg, const PatchDev *__
                                                       BatchFlags f, int m, double rtol) {
   const int p = blockIdx.x;
   if (!f.sol[p]) return;
-  const double s = patch_sum(sg, f.part, p, vec_blocks(pd[p]));
+  const double s = patch_sum(sg, f.part, p, row_blocks(pd[p]));
   if (threadIdx.x == 0) {
     const double beta = sqrt(s);
     const double rr = beta / f.bn[p];
@@ -375,22 +386,12 @@ __global__ __launch_bounds__(256) void kb_set_v(Seg sg, const PatchDev *__restri
 // w = K t (padding rows: 0)
 __global__ __launch_bounds__(256) void kb_spmv_t(Seg sg, const PatchDev *__restrict__ pd,
                                                  const uint8_t *__restrict__ mask) {
-  const VecAt at = vec_at(sg);
-  if (!mask[at.p]) return;
-  const PatchDev &d = pd[at.p];
-  const int64_t R = at.t;
-  if (R >= d.nt * TILE) return;
-  double s = 0.0;
-  if (R < d.nx) {
-    const int64_t q = R / d.ndf;
-    const int r = (int)(R % d.ndf), bb = d.ndf * d.ndf;
-    for (int32_t k = d.rowptr[q]; k < d.rowptr[q + 1]; ++k) {
-      const double *blk = d.bsr + (int64_t)k * bb + r * d.ndf;
-      const double *tv = d.t + (int64_t)d.colidx[k] * d.ndf;
-      for (int c = 0; c < d.ndf; ++c) s = fma(blk[c], tv[c], s);
-    }
-  }
-  d.w[R] = s;
+  const int p = sg.map[blockIdx.x];
+  if (!mask[p]) return;
+  const PatchDev &d = pd[p];
+  const int64_t R = (int64_t)(blockIdx.x - sg.blk0[p]) * 32 + (threadIdx.x >> 3);
+  const double s = row_spmv(d, d.t, R);
+  if ((threadIdx.x & 7) == 0) d.w[R] = s;
 }
 
 // part2[i][block] = partial <V_i, w>, i <= j (blockIdx.y = i)
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__re
   __shared__ int bad;
   const int p = blockIdx.x;
   if (!f.sol[p]) return;
-  const double s = patch_sum(sg, f.part, p, vec_blocks(pd[p]));
+  const double s = patch_sum(sg, f.part, p, row_blocks(pd[p]));
   if (threadIdx.x == 0) {
     const double rr = sqrt(s) / f.bn[p];
     f.relres[p] = rr;
@@ -730,8 +731,8 @@ void b_solve_begin(BatchPlan &B) {
 void b_cycle_begin(BatchPlan &B) {
   const BatchFlags &f = B.f;
   const unsigned nv = B.vec.nblk;
-  hipLaunchKernelGGL(kb_resid, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol, f.part);
-  hipLaunchKernelGGL(kb_cycle_start, dim3(B.P), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.m,
+  hipLaunchKernelGGL(kb_resid, dim3(B.row.nblk), dim3(256), 0, B.stream, B.row, B.d_pd, f.sol, f.part);
+  hipLaunchKernelGGL(kb_cycle_start, dim3(B.P), dim3(256), 0, B.stream, B.row, B.d_pd, f, B.m,
                      B.rtol);
   hipLaunchKernelGGL(kb_set_v, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon, f.scale, 0);
   MAFEM_HIP(hipGetLastError());
@@ -742,7 +743,7 @@ void b_cycle_steps(BatchPlan &B, int j0, int j1) {
   const unsigned nv = B.vec.nblk;
   for (int j = j0; j < j1; ++j) {
     b_lu_solve(B, f.kon);
-    hipLaunchKernelGGL(kb_spmv_t, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon);
+    hipLaunchKernelGGL(kb_spmv_t, dim3(B.row.nblk), dim3(256), 0, B.stream, B.row, B.d_pd, f.kon);
     for (int pass = 0; pass < 2; ++pass) {  // classical Gram-Schmidt, twice
       hipLaunchKernelGGL(kb_mdot, dim3(nv, j + 1), dim3(256), 0, B.stream, B.vec, B.d_pd, f.kon,
                          f.part2);
@@ -769,8 +770,8 @@ void b_cycle_end(BatchPlan &B) {
   hipLaunchKernelGGL(kb_vcomb, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.m);
   b_lu_solve(B, f.sol);
   hipLaunchKernelGGL(kb_add_t, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol);
-  hipLaunchKernelGGL(kb_resid, dim3(nv), dim3(256), 0, B.stream, B.vec, B.d_pd, f.sol, f.part);
-  hipLaunchKernelGGL(kb_cycle_end, dim3(B.P), dim3(256), 0, B.stream, B.vec, B.d_pd, f, B.rtol);
+  hipLaunchKernelGGL(kb_resid, dim3(B.row.nblk), dim3(256), 0, B.stream, B.row, B.d_pd, f.sol, f.part);
+  hipLaunchKernelGGL(kb_cycle_end, dim3(B.P), dim3(256), 0, B.stream, B.row, B.d_pd, f, B.rtol);
   hipLaunchKernelGGL(kb_count_sol, dim3(1), dim3(256), 0, B.stream, B.P, f);
   MAFEM_HIP(hipGetLastError());
 }
