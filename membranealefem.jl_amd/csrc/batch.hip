@@ -9,10 +9,8 @@
 // graphs stay valid for every iteration and step.
 #include <algorithm>
 #include <cmath>
-#include <cstdlib>
 #include <cstring>
 #include <new>
-#include <numeric>
 #include <string>
 #include <vector>
 
@@ -35,7 +33,7 @@ struct mafem_batch {
   std::vector<void *> owned;   // device allocations of the plan (rebuilt with it)
   std::vector<void *> fowned;  // device allocations of the flags (live with the batch)
   std::vector<int> prec;       // factor storage precision of each member
-  std::vector<const void *> store;  // where each member's factors lie
+  std::vector<uint64_t> store;      // generation of each member's factor storage
   std::vector<uint8_t> h_fac;  // members known to be flagged for factorization
   mafem_batch_stats stats{};
 };
@@ -161,7 +159,7 @@ void build_plan(mafem_batch &b) {
   b.store.resize(P);
   for (int p = 0; p < P; ++p) {
     const Ctx &c = *ctx[p];
-    b.store[p] = nd_store(c);
+    b.store[p] = nd_generation(c);
     b.h_pd[p] = describe(c);
     b.h_pd[p].prec = b.prec[p];
     b.h_pd[p].V = balloc<double>(b, (B.m + 1) * c.nt * (int64_t)TILE);
@@ -256,7 +254,7 @@ void ensure_hist(mafem_batch &b, int max_iter) {
 bool plan_stale(const mafem_batch &b) {
   for (size_t p = 0; p < b.members.size(); ++p) {
     const Ctx &c = b.members[p]->c;
-    if (nd_store(c) != b.store[p] || nd_prec(c) != b.prec[p]) return true;
+    if (nd_generation(c) != b.store[p] || nd_prec(c) != b.prec[p]) return true;
   }
   return false;
 }

@@ -319,11 +319,11 @@ void b_solve_end(BatchPlan &B);    // unconverged solves: refactor and redo, or 
 void b_update(BatchPlan &B);       // refactor policy, state update, ε, Newton flags, counts
 void b_mark_factored(BatchPlan &B);
 void b_count(BatchPlan &B);        // count[0] = on, count[2] = on && fac
-// fronts of every member in the given precisions, side by side; nd_store: where a
-// context's factors lie (null: nowhere yet)
+// fronts of every member in the given precisions, side by side; nd_generation: how
+// often a context's factor storage has been allocated
 NdBatch *nd_batch_create(Ctx *const *members, const int *prec, int n);
 void nd_batch_free(NdBatch *B);
-const void *nd_store(const Ctx &c);
+uint64_t nd_generation(const Ctx &c);
 
 // Serialises graph recording against context creation on other host threads
 // (creation makes synchronous null-stream copies, which would invalidate a
