@@ -307,8 +307,10 @@ __global__ __launch_bounds__(256) void kb_solve_begin_fin(Seg sg, const PatchDev
   if (threadIdx.x == 0) {
     f.bn[p] = sqrt(s);
     f.kits[p] = 0;
-    f.relres[p] = 0.0;
-    f.sol[p] = s > 0.0 ? 1 : 0;  // a zero right-hand side is solved by x = 0
+    // a zero right-hand side is solved by x = 0; one without a finite norm (an
+    // undefined or overflowed state) has no solve, and relres says so to the update
+    f.relres[p] = isfinite(s) ? 0.0 : s;
+    f.sol[p] = s > 0.0 && isfinite(s) ? 1 : 0;
   }
 }
 
@@ -521,12 +523,9 @@ __global__ __launch_bounds__(256) void kb_add_t(Seg sg, const PatchDev *__restri
   if (at.t < d.nt * TILE) d.x[at.t] += d.t[at.t];
 }
 
-// after a cycle: the true relative residual decides; converged solves leave sol,
-// and where the factors were singular (an infinite or undefined residual) the
-// next attempt starts from zero again
+// after a cycle: the true relative residual decides; converged solves leave sol
 __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__restrict__ pd,
                                                     BatchFlags f, double rtol) {
-  __shared__ int bad;
   const int p = blockIdx.x;
   if (!f.sol[p]) return;
   const double s = patch_sum(sg, f.part, p, row_blocks(pd[p]));
@@ -534,11 +533,7 @@ __global__ __launch_bounds__(256) void kb_cycle_end(Seg sg, const PatchDev *__re
     const double rr = sqrt(s) / f.bn[p];
     f.relres[p] = rr;
     if (rr <= rtol) f.sol[p] = 0;
-    bad = isfinite(rr) ? 0 : 1;
   }
-  __syncthreads();
-  if (bad)
-    for (int64_t t = threadIdx.x; t < pd[p].nt * TILE; t += 256) pd[p].x[t] = 0.0;
 }
 
 // count[5] = Arnoldi processes still running
@@ -615,6 +610,16 @@ __global__ __launch_bounds__(256) void kb_solve_end(int P, const PatchDev *__res
   }
 }
 
+// a solve that goes on after singular factors (an infinite or undefined
+// residual) starts from zero again; one that was given up keeps what it has
+__global__ __launch_bounds__(256) void kb_drop_x(Seg sg, const PatchDev *__restrict__ pd,
+                                                 BatchFlags f) {
+  const VecAt at = vec_at(sg);
+  if (!f.sol[at.p] || isfinite(f.relres[at.p])) return;
+  const PatchDev &d = pd[at.p];
+  if (at.t < d.nt * TILE) d.x[at.t] = 0.0;
+}
+
 __global__ __launch_bounds__(256) void kb_mark_factored(int P, BatchFlags f) {
   for (int p = threadIdx.x; p < P; p += 256)
     if (f.on[p] && f.fac[p]) {
@@ -683,15 +688,16 @@ __global__ __launch_bounds__(256) void kb_sumsq_x(Seg sg, const PatchDev *__rest
   if (threadIdx.x == 0) part[blockIdx.x] = a;
 }
 
-// ε = |Δu|_2 / nmdf (FiniteElement.jl:48); a patch stops when ε < εnr
-// (:54), when ε is not finite, or after max_iter iterations
+// ε = |Δu|_2 / nmdf (FiniteElement.jl:48), undefined where the solve ended
+// without a finite residual; a patch stops when ε < εnr (:54), when ε is not
+// finite, or after max_iter iterations
 __global__ __launch_bounds__(256) void kb_newton_check(Seg sg, const PatchDev *__restrict__ pd,
                                                        BatchFlags f, int max_iter) {
   const int p = blockIdx.x;
   if (!f.on[p]) return;
   const double s = patch_sum(sg, f.part, p, vec_blocks(pd[p]));
   if (threadIdx.x == 0) {
-    const double eps = sqrt(s) / pd[p].nmdf;
+    const double eps = isfinite(f.relres[p]) ? sqrt(s) / pd[p].nmdf : __builtin_nan("");
     const int it = f.iters[p];
     f.eps_hist[(int64_t)p * max_iter + it] = eps;
     f.eps[p] = eps;
@@ -778,6 +784,7 @@ void b_cycle_end(BatchPlan &B) {
 
 void b_solve_end(BatchPlan &B) {
   hipLaunchKernelGGL(kb_solve_end, dim3(1), dim3(256), 0, B.stream, B.P, B.d_pd, B.f);
+  hipLaunchKernelGGL(kb_drop_x, dim3(B.vec.nblk), dim3(256), 0, B.stream, B.vec, B.d_pd, B.f);
   MAFEM_HIP(hipGetLastError());
 }
 
