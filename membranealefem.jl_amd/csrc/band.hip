@@ -820,8 +820,8 @@ __device__ __forceinline__ void blk_mm(typename Mfma<S>::V &acc, const S (&a)[4]
   for (int kk = 0; kk < 4; ++kk) acc = Mfma<S>::run(sg * a[kk], b[kk], acc);
 }
 
-// Inverses of the factors of a 64x64 diagonal tile in LDS (row i of P A = L U
-// at st[prow[i]]: L unit lower below the diagonal, U upper), in 16 x 16 blocks: the eight diagonal blocks by
+// Inverses of the factors of a 64x64 diagonal tile in LDS (rows in pivot order) as
+// block products, for the FP32 factors of batches: the eight diagonal blocks by
 // substitution with the row broadcast of v_fmac_f64, four to a wavefront (X =
 // L^-1 on wavefront 0, Y = U^-1 on 1); then, on the matrix cores, the
 // off-diagonal blocks of the 32 x 32 halves (X_10, X_32, Y_01, Y_23, one a
@@ -829,26 +829,17 @@ __device__ __forceinline__ void blk_mm(typename Mfma<S>::V &acc, const S (&a)[4]
 // wavefront), X_lower = -X_bb (L_ba X_aa).  A wavefront loads all operands of
 // a stage before its first product.  Li and Ui receive the inverses as full
 // row-major tiles (zeros outside the triangles, ones on L^-1's diagonal).  256
-// threads; st is overwritten.  10.9 k cycles a tile, against 29.8 k for
-// column sweeps in LDS and one block row a round and 21 k for tri_inv_sub,
-// whose smaller residuals are not worth it here, in the factorization's chain
-// (64x64 ALEVB 16.3 -> 17.6 ms a step for the same refinement sweeps).
+// threads; st is overwritten.  8.3 k cycles a tile in FP32 with the rows' move into
+// pivot order, against 9.0 k for tri_inv, whose residuals are 3 to 30 times smaller: what
+// these factors do not precondition a batch solves with FP64 ones, and which patches
+// move there (mafem_batch_stats.fp64_patches) stays as it was.
 template <class S>
-__device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *__restrict__ Li,
-                                            S *__restrict__ Ui) {
+__device__ __forceinline__ void tri_inv_products(S (*st)[T + 1], S *__restrict__ Li,
+                                                 S *__restrict__ Ui) {
   using V = typename Mfma<S>::V;
   const int lane = (int)threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int cc = lane & 15, g = lane >> 4;
-  {  // rows into pivot order
-    S v[T / 4];
-#pragma unroll
-    for (int it = 0; it < T / 4; ++it) v[it] = st[prow[4 * it + w]][lane];
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = v[it];
-    __syncthreads();
-  }
   if (w < 2) {
     // a 16-lane row per diagonal block: lane = row of the triangle and column
     // of its inverse; U_bb with rows and columns reversed (a lower triangle
@@ -938,127 +929,171 @@ __device__ __forceinline__ void tri_inv_lds(S (*st)[T + 1], const int *prow, S *
   }
 }
 
-// v of lane row 0, 1, 2, 3 of the wavefront (16 lanes each), delivered to every
-// lane row (gfx950's row swaps: three for the four values of a 32-bit word)
-__device__ __forceinline__ void rows_all(unsigned v, unsigned (&o)[4]) {
-  const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
-  o[0] = a[0];
-  o[1] = a[1];
-  o[2] = b[0];
-  o[3] = b[1];
-}
-__device__ __forceinline__ void rows_all(float v, float (&o)[4]) {
-  unsigned u[4];
-  rows_all(__float_as_uint(v), u);
-#pragma unroll
-  for (int g = 0; g < 4; ++g) o[g] = __uint_as_float(u[g]);
-}
-__device__ __forceinline__ void rows_all(double v, double (&o)[4]) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  unsigned lo[4], hi[4];
-  rows_all((unsigned)u, lo);
-  rows_all((unsigned)(u >> 32), hi);
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-    o[g] = __longlong_as_double((long long)(((unsigned long long)hi[g] << 32) | lo[g]));
-}
-// accumulator row acc_row(q) of lane row g as an index into a column's 16 rows
-template <class S>
-__host__ __device__ constexpr int acc_idx(int g, int q) {
-  return sizeof(S) == 8 ? g + 4 * q : 4 * g + q;
-}
-
-// Block column J of Z = G^-1 by one wavefront, G lower triangular in 16 x 16
-// blocks with entry (i, k) at G[i si + k sk] (L itself, or U transposed) and rd
-// its diagonal's reciprocals (LOW: a unit diagonal): Z_IJ = G_II^-1 (-sum_{J <=
-// k < I} G_Ik Z_kJ).  The sums run on the matrix cores, each row's term as soon
-// as its Z_kJ is there; a diagonal block is solved by substitution
-// (unit_solve16, its rows scaled to a unit diagonal), one of Z's columns a
-// lane, every lane row alike.  Entry (i, j) of Z goes to Z[i zi + j zj], zeros
-// above the diagonal block too.
+// One factor of tri_inv, seen as the lower triangle G of a tile in LDS: entry (i,
+// k) of G at st[i SI + k SK], L itself or U transposed.
 template <class S, bool LOW>
-__device__ __forceinline__ void tri_inv_col(int J, const S *G, int si, int sk, const S *rd,
-                                            S *__restrict__ Z, int zi, int zj) {
+struct TriInv {
   using V = typename Mfma<S>::V;
-  const int cc = (int)threadIdx.x & 15, g = ((int)threadIdx.x & 63) >> 4;
-  V t[4];
+  static constexpr int SI = LOW ? T + 1 : 1, SK = LOW ? 1 : T + 1;
+
+  // entry (r, c) of a diagonal block, of G or of its inverse
+  static __device__ __forceinline__ S tri(S v, int r, int c) {
+    return LOW && r == c ? S(1) : ((LOW ? r > c : r >= c) ? v : S(0));
+  }
+  // the matrix cores' operands of a 16 x 16 block, four entries a lane: as A, row
+  // lane % 16 and column acc_row(kk); as B, row acc_row(kk) and column lane % 16 (an
+  // accumulator's own layout, so that a product can be the next one's B)
+  static __device__ __forceinline__ void load_a(S (&v)[4], const S *st, int i, int k) {
+    const int cc = (int)threadIdx.x & 15;
+    const S *p = st + (16 * i + cc) * SI + 16 * k * SK;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) t[i] = V{0, 0, 0, 0};
+    for (int q = 0; q < 4; ++q) v[q] = p[acc_row<S>(q) * SK];
+    if (i == k)
 #pragma unroll
-  for (int I = 0; I < 4; ++I) {
-    S *out = Z + 16 * I * zi + (16 * J + cc) * zj;
-    if (I < J) {
+      for (int q = 0; q < 4; ++q) v[q] = tri(v[q], cc, acc_row<S>(q));
+  }
+  template <int SG>
+  static __device__ __forceinline__ void mm(V &acc, const S (&a)[4], const V &b) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) out[acc_row<S>(q) * zi] = S(0);
-      continue;
-    }
-    // lane row entries: -(row cc of the unit triangle), operands of the rows below
-    const S rc = LOW ? S(1) : rd[16 * I + cc];
-    S m[16], x[16], a[3][4];
+    for (int q = 0; q < 4; ++q) acc = Mfma<S>::run(SG < 0 ? -a[q] : a[q], b[q], acc);
+  }
+
+  // The diagonal blocks' inverses in place by one wavefront, a 16-lane row each
+  // (lane: row of the triangle, scaled to a unit diagonal, and column of the inverse)
+  static __device__ __forceinline__ void diag(S *st) {
+    const int cc = (int)threadIdx.x & 15, g = ((int)threadIdx.x & 63) >> 4;
+    S *blk = st + 16 * g * (T + 2);
+    S m[16], x[16];
 #pragma unroll
-    for (int k = 0; k < 15; ++k) m[k] = G[(16 * I + cc) * si + (16 * I + k) * sk];
-#pragma unroll
-    for (int i = I + 1; i < 4; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        a[i - 1][q] = -G[(16 * i + cc) * si + (16 * I + acc_row<S>(q)) * sk];
+    for (int k = 0; k < 15; ++k) m[k] = blk[cc * SI + k * SK];
+    const S rc = LOW ? S(1) : S(1) / blk[cc * SI + cc * SK];
 #pragma unroll
     for (int k = 0; k < 15; ++k) m[k] *= -rc;
-    if (I == J) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = i == cc ? rc : S(0);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        S r4[4];
-        rows_all(LOW ? t[I][q] : t[I][q] * rd[16 * I + acc_row<S>(q)], r4);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) x[acc_idx<S>(h, q)] = r4[h];
-      }
-    }
+    for (int i = 0; i < 16; ++i) x[i] = i == cc ? rc : S(0);
     settle(m);
     unit_solve16<0>(x, m);
-    S z[4];  // rows acc_row(q): the lane's part of the result, and of a B operand
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (LOW ? i > cc : i >= cc) blk[i * SI + cc * SK] = x[i];
+  }
+
+  // Block column J of Z = G^-1 below its diagonal block, in registers: Z_IJ = G_II^-1
+  // t, t = -sum_{J <= k < I} G_Ik Z_kJ, with the inverse of G_II, for U with one
+  // correction by the residual t - G_II Z_IJ (d: the diagonal blocks before diag; L's
+  // entries are at most 1 and its blocks well conditioned: correcting X too changes
+  // no residual)
+  template <int J>
+  static __device__ __forceinline__ void column(const S *st, const S (&d)[4][4], V (&z)[4]) {
+    const int cc = (int)threadIdx.x & 15;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const S lo = g & 1 ? x[acc_idx<S>(1, q)] : x[acc_idx<S>(0, q)];
-      const S hi = g & 1 ? x[acc_idx<S>(3, q)] : x[acc_idx<S>(2, q)];
-      z[q] = g & 2 ? hi : lo;
+      const int r = acc_row<S>(q);
+      z[J][q] = tri(st[16 * J * (T + 2) + r * SI + cc * SK], r, cc);
     }
 #pragma unroll
-    for (int i = I + 1; i < 4; ++i)
+    for (int I = J + 1; I < 4; ++I) {
+      S inv[4];
+      load_a(inv, st, I, I);
+      V t = V{0, 0, 0, 0}, y = t;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) t[i] = Mfma<S>::run(a[i - 1][q], z[q], t[i]);
+      for (int k = J; k < I; ++k) {
+        S a[4];
+        load_a(a, st, I, k);
+        mm<-1>(t, a, z[k]);
+      }
+      mm<1>(y, inv, t);
+      if constexpr (!LOW) {
+        mm<-1>(t, d[I], y);
+        mm<1>(y, inv, t);
+      }
+      z[I] = y;
+    }
+  }
+  template <int J>
+  static __device__ __forceinline__ void store(S *st, const V (&z)[4]) {
+    const int cc = (int)threadIdx.x & 15;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) out[acc_row<S>(q) * zi] = z[q];
+    for (int I = J + 1; I < 4; ++I)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) st[(16 * I + acc_row<S>(q)) * SI + (16 * J + cc) * SK] = z[I][q];
+  }
+
+  // part 0: block column 0 (15 products for U, 9 for L), part 1: block columns 1 and 2
+  // (13 and 7)
+  static __device__ __forceinline__ void run(S *st, int part) {
+    S d[4][4];
+    if constexpr (!LOW)
+#pragma unroll
+      for (int I = 1; I < 4; ++I) load_a(d[I], st, I, I);
+    __syncthreads();
+    if (part == 0) diag(st);
+    __syncthreads();
+    V z[4], z2[4];
+    if (part == 0) column<0>(st, d, z);
+    else {
+      column<1>(st, d, z);
+      column<2>(st, d, z2);
+    }
+    __syncthreads();  // every operand has been read
+    if (part == 0) store<0>(st, z);
+    else {
+      store<1>(st, z);
+      store<2>(st, z2);
+    }
+  }
+};
+
+// Inverses of the factors of a 64x64 diagonal tile in LDS (rows in pivot order: L
+// unit lower below the diagonal, U upper), in place, in 16 x 16 blocks: X with L X
+// = I and Y with Y U = I, to the residual of substitution, which is what their uses
+// need (U12 = X A12 leaves L U12 - A12 = (L X - I) A12, L21 = A21 Y leaves A21 (Y U -
+// I)).  Wavefronts 0 and 2 form X, 1 and 3 Y^T = (U^T)^-1.  Block products without
+// the correction multiply the residual by the diagonal blocks' condition, and Y
+// from U Y = I by U's: 10.7 k cycles a tile (FP32 8.3 k) against 12.2 k (9.0 k) here,
+// but a solve without refinement left 3 to 30 times as much (96x80 LAG 1.3e-10
+// against 1.3e-11, 64x64 EUL 2.6e-7 against 3.1e-8), and FGMRES on FP32 factors
+// took 20 to 70 % more steps or did not converge (64x64 EUL).  Substitution in every
+// block leaves the same residuals in 19.7 k cycles.  Li and Ui receive full row-major
+// tiles (zeros outside the triangles, ones on L^-1's diagonal).  256 threads; st is
+// overwritten.
+template <class S>
+__device__ __forceinline__ void tri_inv(S (*st)[T + 1], S *__restrict__ Li, S *__restrict__ Ui) {
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (w & 1) TriInv<S, false>::run(&st[0][0], w >> 1);
+  else TriInv<S, true>::run(&st[0][0], w >> 1);
+  __syncthreads();
+#pragma unroll 4
+  for (int it = 0; it < T * T / 256; ++it) {
+    const int e = it * 256 + (int)threadIdx.x, r = e / T, c = e % T;
+    const S v = st[r][c];
+    Li[e] = r > c ? v : (r == c ? S(1) : S(0));
+    Ui[e] = r <= c ? v : S(0);
   }
 }
 
-// Inverses of the factors of a 64x64 diagonal tile in LDS (rows in pivot order:
-// L unit lower below the diagonal, U upper) as X with L X = I and Y with Y U = I,
-// the block columns of X and of Y^T independent of each other: wavefronts 0
-// and 1 take X's (0 and 3, 1 and 2), 2 and 3 Y's.  For the band's pass over all
-// tiles after the factorization, in parallel and off its chain: against
-// tri_inv_lds' block products the residual of a solve is up to 20 times smaller
-// (17x13 ALEVB 7e-14 -> 1.5e-14, in FP32 5e-5 -> 2.4e-6), which saves refinement
-// sweeps and Krylov steps (17x13 ALEVB 4.67 -> 4.44 ms a step, 16 patches with FP32
-// factors 55.4 -> 50.4 ms).  Li and Ui receive full row-major tiles (zeros
-// outside the triangles, ones on L^-1's diagonal).  256 threads; rd: T entries
-// of LDS.
+// Inverses of the tile that diag_mm_lds left in its LDS buffer (row i of P A = L U
+// at st[prow[i]]); batch: FP32 factors by tri_inv_products
 template <class S>
-__device__ __forceinline__ void tri_inv_sub(S (*st)[T + 1], S *rd, S *__restrict__ Li,
-                                            S *__restrict__ Ui) {
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  if (threadIdx.x < T) rd[threadIdx.x] = S(1) / st[threadIdx.x][threadIdx.x];
+__device__ __forceinline__ void tri_inv_lds(S *lds, S *__restrict__ Li, S *__restrict__ Ui,
+                                            bool batch) {
+  S(*st)[T + 1] = reinterpret_cast<S(*)[T + 1]>(lds);
+  const int *prow = lu_prow(lds);
+  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  S v[T / 4];
+#pragma unroll
+  for (int it = 0; it < T / 4; ++it) v[it] = st[prow[4 * it + w]][lane];
   __syncthreads();
-#pragma unroll 1
-  for (int h = 0; h < 2; ++h) {
-    const int J = w & 1 ? 1 + h : 3 * h;
-    if (w < 2) tri_inv_col<S, true>(J, &st[0][0], T + 1, 1, rd, Li, T, 1);
-    else tri_inv_col<S, false>(J, &st[0][0], 1, T + 1, rd, Ui, 1, T);
+#pragma unroll
+  for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = v[it];
+  __syncthreads();
+  if constexpr (sizeof(S) == 4) {
+    if (batch) {
+      tri_inv_products<S>(st, Li, Ui);
+      return;
+    }
   }
+  tri_inv<S>(st, Li, Ui);
 }
 
 // diagonal LU of tile (K, K) of a band by a 256-thread block
@@ -1478,13 +1513,13 @@ __global__ void k_span_init(unsigned long long *__restrict__ span) {
 template <class S>
 __device__ __forceinline__ void tile_inv_body(int64_t I, int tb, const S *__restrict__ band,
                                               S *__restrict__ linv, S *__restrict__ uinv) {
-  __shared__ S st[T][T + 1], rd[T];
+  __shared__ S st[T][T + 1];
   const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
   const S *D = tile_ptr(band, tb, I, I);
 #pragma unroll
   for (int it = 0; it < T / 4; ++it) st[4 * it + w][lane] = D[(4 * it + w) * T + lane];
   __syncthreads();
-  tri_inv_sub<S>(st, rd, linv + I * T * T, uinv + I * T * T);
+  tri_inv<S>(st, linv + I * T * T, uinv + I * T * T);
 }
 
 template <class S>
