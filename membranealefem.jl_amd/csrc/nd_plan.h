@@ -210,14 +210,14 @@ inline double plan_cost(int64_t n1, int64_t n2, int ndf, int leaf) {
   return 33.0 * s + products * 2.0 * NT * NT * NT / 45e6;
 }
 
-// The leaf size of least cost.  Larger leaves save levels but lengthen the
+// The leaf size of least cost, at most `most`.  Larger leaves save levels but lengthen the
 // leaf's own chain and cost products.  A time step with leaves of 4 and with the
 // size taken: 10x10 LAG 1.83 and 1.47 ms, 24x10 EUL 2.69 and 2.41, 96x80 LAG 11.68
 // and 11.15; 64x64 ALEVB stays at 4 (17.6 ms with 7, 16.3 with 4).
-inline int choose_leaf(int64_t n1, int64_t n2, int ndf) {
+inline int choose_leaf(int64_t n1, int64_t n2, int ndf, int most = 10) {
   int best = 4;
   double least = plan_cost(n1, n2, ndf, best);
-  for (int leaf = 5; leaf <= 10; ++leaf) {
+  for (int leaf = 5; leaf <= most; ++leaf) {
     const double c = plan_cost(n1, n2, ndf, leaf);
     if (c < least) {
       least = c;
