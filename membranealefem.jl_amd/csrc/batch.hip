@@ -159,7 +159,7 @@ void build_plan(mafem_batch &b) {
   b.store.resize(P);
   for (int p = 0; p < P; ++p) {
     const Ctx &c = *ctx[p];
-    b.store[p] = nd_generation(c);
+    b.store[p] = nd_batch_generation(c);
     b.h_pd[p] = describe(c);
     b.h_pd[p].prec = b.prec[p];
     b.h_pd[p].V = balloc<double>(b, (B.m + 1) * c.nt * (int64_t)TILE);
@@ -249,12 +249,12 @@ void ensure_hist(mafem_batch &b, int max_iter) {
   B.f.eps_hist = falloc<double>(b, (int64_t)B.P * max_iter);
 }
 
-// The plan is stale when a member's factor storage moved (a precision change
-// through its own solver entry points).
+// The plan is stale when a member's factor storage moved (another batch that it is
+// in has it in another precision).
 bool plan_stale(const mafem_batch &b) {
   for (size_t p = 0; p < b.members.size(); ++p) {
     const Ctx &c = b.members[p]->c;
-    if (nd_generation(c) != b.store[p] || nd_prec(c) != b.prec[p]) return true;
+    if (nd_batch_generation(c) != b.store[p] || nd_batch_prec(c) != b.prec[p]) return true;
   }
   return false;
 }
@@ -431,7 +431,7 @@ int mafem_batch_create(mafem_batch **out, int32_t n, mafem_ctx *const *members,
       std::vector<uint8_t> fac(n);
       for (int32_t i = 0; i < n; ++i) {
         const Ctx &c = members[i]->c;
-        fac[i] = (c.batch_factor_prec == b.prec[i] && nd_prec(c) == b.prec[i]) ? 0 : 1;
+        fac[i] = (c.batch_factor_prec == b.prec[i] && nd_batch_prec(c) == b.prec[i]) ? 0 : 1;
       }
       b.h_fac = fac;
       MAFEM_HIP(hipMemcpy(b.B.f.fac, fac.data(), n, hipMemcpyHostToDevice));
@@ -489,14 +489,14 @@ int mafem_batch_time_step(mafem_batch *bp, const double *time, const double *dt,
     const int P = B.P;
     for (mafem_ctx *m : b.members) {
       MAFEM_HIP(hipStreamSynchronize(m->c.stream));
-      // the batch factors into the member's fronts: a factorization the context
-      // kept there for its own Krylov solves is gone
+      // the step moves the member on: a factorization that the context kept for its
+      // own Krylov solves belongs to an old tangent
       m->c.have_factor = false;
     }
     if (plan_stale(b)) build_plan(b);
     ensure_hist(b, max_iter);
     BatchFlags &f = B.f;
-    // and a member that has factored for itself since is factored afresh
+    // a member whose storage another batch had allocated afresh is factored again
     const uint8_t one = 1;
     for (int p = 0; p < P; ++p)
       if (b.members[p]->c.batch_factor_prec != b.prec[p] && !b.h_fac[p])

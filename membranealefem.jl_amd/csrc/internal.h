@@ -149,7 +149,7 @@ struct Ctx {
   mafem_stats stats{};
   int32_t n_band_solve = 0;     // running count of triangular-solve sweeps
 
-  // factorization left in the fronts by a batch (kept when the context joins
+  // factorization left in its fronts by a batch (kept when the context joins
   // another batch): its precision, 0 = none; batch_prec = precision a batch
   // last chose for this context (an FP64 fallback stays FP64)
   int batch_factor_prec = 0;
@@ -319,11 +319,13 @@ void b_solve_end(BatchPlan &B);    // unconverged solves: refactor and redo, or 
 void b_update(BatchPlan &B);       // refactor policy, state update, ε, Newton flags, counts
 void b_mark_factored(BatchPlan &B);
 void b_count(BatchPlan &B);        // count[0] = on, count[2] = on && fac
-// fronts of every member in the given precisions, side by side; nd_generation: how
-// often a context's factor storage has been allocated
+// fronts of every member in the given precisions, side by side; nd_batch_prec,
+// nd_batch_generation: precision of a context's factor storage for batches (0: none) and
+// how often it has been allocated
 NdBatch *nd_batch_create(Ctx *const *members, const int *prec, int n);
 void nd_batch_free(NdBatch *B);
-uint64_t nd_generation(const Ctx &c);
+int nd_batch_prec(const Ctx &c);
+uint64_t nd_batch_generation(const Ctx &c);
 
 // Serialises graph recording against context creation on other host threads
 // (creation makes synchronous null-stream copies, which would invalidate a
@@ -351,7 +353,7 @@ void band_solve(Ctx &c, const double *d_rhs, double *d_x);
 // nested-dissection fronts (band.hip; band_fill / band_factor / band_solve
 // route to them when Ctx::ordering is 1)
 void nd_free(Ctx &c);
-int nd_prec(const Ctx &c);       // storage precision of the fronts (0: none)
+int nd_prec(const Ctx &c);       // storage precision of the context's own factors (0: none)
 int nd_fronts(const Ctx &c);     // fronts of the elimination tree (0: not built)
 int nd_steps(const Ctx &c);      // dependent tile steps of one factorization
 double nd_flops(const Ctx &c);   // algorithmic FLOPs of one factorization
@@ -365,7 +367,6 @@ struct NdSpans {
 void nd_begin_spans(Ctx &c);
 void nd_end_spans(Ctx &c);
 bool nd_read_spans(Ctx &c, NdSpans &step, NdSpans &schur);
-int64_t nd_bytes(const Ctx &c);  // bytes of factor storage
 void bsr_spmv(Ctx &c, const double *d_x, double *d_y, const double *d_b = nullptr);
 void vec_axpby(Ctx &c, int64_t n, double a, const double *x, double b, double *y);
 void vec_zero(Ctx &c, int64_t n, double *y);
