@@ -227,6 +227,21 @@ inline int choose_leaf(int64_t n1, int64_t n2, int ndf, int most = 10) {
   return best;
 }
 
+// What keeping M = L21 W and N = Z U12 of every front saves, in microseconds, over a
+// factorization in `prec` bits and `solves` solves with it.  A solve has one launch up
+// and one down a level instead of two each, 4.5 a level below the root; forming the two
+// takes their products at 45 TFLOP/s (half in FP32) and 3 a level.  Time steps without
+// and with them, in ms: 24x24 LAG 2.14 and 2.13, 40x40 LAG 3.60 and 3.52, 48x48 LAG 5.41
+// and 5.35, 32x32 EUL 4.34 and 4.31; where this says no, 56x56 LAG 6.51 and 6.59, 40x40 EUL
+// 5.44 and 5.49, 24x24 ALEVB 3.28 and 3.36, 48x48 ALEVB 10.2 and 10.6; with FGMRES on FP32
+// factors 32x32 ALEVB 5.26 and 5.05, 48x48 LAG 8.3 and 7.6.
+inline double mn_saving(const Plan &P, double solves, int prec) {
+  double products = 0.0;
+  for (const Front &F : P.fr) products += (double)(F.FT - F.fT) * F.fT * (F.fT + 1);
+  const double form = products * 2.0 * NT * NT * NT / 45e6;
+  return solves * 4.5 * (P.levels - 1) - (3.0 * P.levels + (prec == 32 ? 0.5 * form : form));
+}
+
 // First tile of each front's Schur complement in one pool, and the pool's size.  It
 // is there from the front's level to its parent's; fronts that share both levels
 // lie together, each such group in the lowest gap that is free for its levels.
