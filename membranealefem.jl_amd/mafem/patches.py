@@ -110,26 +110,38 @@ class Patch:
         self.dev.close()
 
 
-def device_bytes(spec: PatchSpec, precision=32, restart=20, ordering="band"):
-    """Device memory of one patch context plus its batch storage (bytes).
-    ordering "nd": its factorization held as nested-dissection fronts (as batches
-    do) instead of a band, bounded by 2.5 times the one-chain band of the same
-    precision and less from 45 nodes a side on (fronts of 16x16, 40x40, 66x66 and
-    96x96 patches measure at most 2.25, 1.75, 1.6 and 1.05 times it)."""
+def _band_tiles(motion, n):
+    """Tile rows and half bandwidth of an n x n patch's band of 64x64 tiles."""
+    ndf = {int(LAG): 4, int(EUL): 7}.get(int(motion), 8)
+    nt = -(-(n + 2) ** 2 * ndf // 64)
+    return nt, min(-(-((2 * (n + 2) + 3) * ndf - 1) // 64), max(1, nt - 1))
+
+
+def front_bytes(spec: PatchSpec, precision=32, own=False):
+    """Bound on a patch's nested-dissection fronts (bytes), as a batch holds them: 2.8
+    times the one-chain band of the same precision (4x4, 11x11 and 12x12 EUL patches hold
+    2.7 to 2.8 times it) and less from 38 nodes a side on.  `own`: as the context's own
+    factorization holds them, 1.5 times that where it may keep the products that
+    shorten its solves (in FP64, with the direct solver, up to 62 elements a side)."""
+    nt, tb = _band_tiles(spec.motion, spec.n)
+    b = min(2.8, max(1.15, 112 / (spec.n + 2))) * nt * (2 * tb + 3) * 64 * 64 * (precision // 8)
+    return int(1.5 * b if own and (precision == 32 or spec.n <= 62) else b)
+
+
+def device_bytes(spec: PatchSpec, precision=32, restart=20, ordering="band", own=False):
+    """Device memory of one patch context plus its batch storage (bytes), its
+    factorization a band or (ordering "nd") the fronts of a batch or of its own."""
     ndf = {int(LAG): 4, int(EUL): 7}.get(int(spec.motion), 8)
     n = spec.n
     numel = n * n
-    n1 = n + 2
-    numnp = n1 * n1
-    nx = numnp * ndf
-    nt = -(-nx // 64)
-    tb = min(-(-((2 * n1 + 3) * ndf - 1) // 64), max(1, nt - 1))
+    numnp = (n + 2) * (n + 2)
+    nt, tb = _band_tiles(spec.motion, n)
     ne = 9 * ndf
     es = 4 if precision == 32 else 8
     rows = nt + tb if nt >= 8 * tb else nt  # the two-ended layout keeps tb more tile rows
     band = rows * (2 * tb + 1) * 64 * 64 * es + 2 * rows * 64 * 64 * es
     if ordering == "nd":
-        band = int(min(2.5, max(1.1, 112 / n1)) * nt * (2 * tb + 3) * 64 * 64 * es)
+        band = front_bytes(spec, precision, own)
     nnzb = numnp * 25
     kel = (numel + 4 * n) * ne * ne * 8
     bsr = nnzb * ndf * ndf * 8

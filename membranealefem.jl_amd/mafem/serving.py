@@ -92,7 +92,8 @@ class Server:
 
     def _bytes(self, r):
         # FP64 storage in the estimate (a member may fall back to it)
-        return int(1.15 * device_bytes(r.spec, precision=64, ordering="nd"))
+        own = r.spec.n * r.spec.n >= self.solo_min_elements
+        return int(1.15 * device_bytes(r.spec, precision=64, ordering="nd", own=own))
 
     def run(self, requests, time_limit=None, log=None):
         """Serve `requests` (sorted by arrival); returns them with results."""
