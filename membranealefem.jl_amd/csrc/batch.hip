@@ -141,6 +141,7 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // allocated once per batch and keep their contents).
 void build_plan(mafem_batch &b) {
   free_plan(b);
+  b.store.assign(b.members.size(), ~0ull);  // stale until complete: an allocation may fail below
   BatchPlan &B = b.B;
   const int P = (int)b.members.size();
   B.P = P;
@@ -156,10 +157,8 @@ void build_plan(mafem_batch &b) {
   } catch (const ArgError &e) {
     throw BatchError{"batch: " + e.msg, e.code};
   }
-  b.store.resize(P);
   for (int p = 0; p < P; ++p) {
     const Ctx &c = *ctx[p];
-    b.store[p] = nd_batch_generation(c);
     b.h_pd[p] = describe(c);
     b.h_pd[p].prec = b.prec[p];
     b.h_pd[p].V = balloc<double>(b, (B.m + 1) * c.nt * (int64_t)TILE);
@@ -198,6 +197,7 @@ void build_plan(mafem_batch &b) {
   B.node = make_seg(b, bn, 256);
   B.f.part = balloc<double>(b, std::max<int64_t>(B.row.nblk, 1));
   B.f.part2 = balloc<double>(b, std::max<int64_t>((int64_t)B.vec.nblk * (B.m + 1), 1));
+  for (int p = 0; p < P; ++p) b.store[p] = nd_batch_generation(*ctx[p]);
 }
 
 // Per-patch flags and Arnoldi state, once per batch.
